@@ -19,23 +19,19 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, ui
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, kRsrcWord3);
 }
 
-// Resource for plane z (clamped into [0, D)) of a volume; `valid == false` gives a zero-sized
-// buffer, so loads through it return 0 and stores through it are dropped. z and valid must be
-// workgroup-uniform; the explicit readfirstlane keeps the address arithmetic on the scalar unit
-// (a clamp that the compiler selects as a VALU op would otherwise force a per-lane loop around
-// every access through the resource).
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_rsrc(const void* vol, int z, int D, int64_t plane_bytes,
-                                                               bool valid) {
-    const int zc = __builtin_amdgcn_readfirstlane(z < 0 ? 0 : (z >= D ? D - 1 : z));
-    const int nb = __builtin_amdgcn_readfirstlane(valid ? (int)plane_bytes : 0);
-    return make_rsrc((const char*)vol + (int64_t)zc * plane_bytes, (uint32_t)nb);
+// The same resource as four plain words, for addresses that advance in place: word 0-1 the address
+// (its upper 16 bits are zero for a device address, which is the stride field of a raw buffer),
+// word 2 the size in bytes (0: loads return 0, stores are dropped), word 3 as above. Built this way
+// a plane's resource costs the two scalar additions that advance its address; through
+// make_buffer_rsrc the compiler masks the address and rebuilds all four words for every access.
+typedef int rsrc_words __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ rsrc_words words_at(uint64_t addr, uint32_t bytes) {
+    return rsrc_words{(int)(uint32_t)addr, (int)(uint32_t)(addr >> 32), (int)bytes, kRsrcWord3};
 }
-
-// Resource for `bytes` bytes at a workgroup-uniform address; `valid == false` gives a zero-sized
-// buffer (the address is then never dereferenced).
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_at(uint64_t addr, uint32_t bytes, bool valid) {
-    return make_rsrc((const void*)(uintptr_t)addr, valid ? bytes : 0u);
-}
+__device__ float raw_load_f32(rsrc_words r, int voff, int soff, int aux) __asm("llvm.amdgcn.raw.buffer.load.f32");
+__device__ unsigned short raw_load_b16(rsrc_words r, int voff, int soff, int aux) __asm("llvm.amdgcn.raw.buffer.load.i16");
+__device__ void raw_store_f32(float v, rsrc_words r, int voff, int soff, int aux) __asm("llvm.amdgcn.raw.buffer.store.f32");
+__device__ void raw_store_b16(unsigned short v, rsrc_words r, int voff, int soff, int aux) __asm("llvm.amdgcn.raw.buffer.store.i16");
 
 // Cache-policy operand of the buffer instructions: 0 = default, kNT = non-temporal (the line is
 // streamed: a store does not displace data that will be read again from the L2, a load marks the
@@ -51,6 +47,14 @@ __device__ __forceinline__ float load_elem(__amdgpu_buffer_rsrc_t r, uint32_t vo
         // the builtin returns the raw 32 bits; reinterpret, do not convert
         return __uint_as_float((uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, (int)voff, 0, AUX));
     }
+}
+
+template <bool BF16, int AUX = 0>
+__device__ __forceinline__ float load_elem(rsrc_words r, uint32_t voff) {
+    if constexpr (BF16)
+        return __uint_as_float((uint32_t)raw_load_b16(r, (int)voff, 0, AUX) << 16);
+    else
+        return raw_load_f32(r, (int)voff, 0, AUX);
 }
 
 template <bool BF16>
@@ -75,6 +79,14 @@ __device__ __forceinline__ void store_elem_buf(__amdgpu_buffer_rsrc_t r, uint32_
     } else {
         __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, (int)voff, 0, AUX);
     }
+}
+
+template <bool BF16, int AUX = 0>
+__device__ __forceinline__ void store_elem_buf(rsrc_words r, uint32_t voff, float v) {
+    if constexpr (BF16)
+        raw_store_b16(f32_to_bf16_bits(v), r, (int)voff, 0, AUX);
+    else
+        raw_store_f32(v, r, (int)voff, 0, AUX);
 }
 
 template <bool BF16>

@@ -68,44 +68,58 @@
 
 namespace fl {
 
-// Loads NV consecutive floats from a 16-byte aligned LDS address: float4s, then a tail of 2 or 1
-// floats as a float2 or a float (a tail of 3 as one more float4, which reads one float past the
-// row; it is not used), row_read(NV) floats in all. Each vector passes through an empty asm
-// operand that needs all of its lanes, so that the loads stay whole: otherwise the optimizer
-// re-partitions them along the box-sums' blocks (a row of 10 floats became b128 + b96 + read2_b32
-// + b32 instead of b128 + b128 + b64), which costs LDS instructions and bank cycles. The 2-float
-// tail (rather than a third float4) also keeps two registers per row free.
+// A row of NV consecutive floats at a 16-byte aligned LDS address, read as float4s, then a tail of 2
+// or 1 floats as a float2 or a float (a tail of 3 as one more float4, which reads one float past the
+// row; it is not used), row_read(NV) floats in all. row_load issues the reads; row_take hands out the
+// values, each vector through an empty asm operand that needs all of its lanes, so that the loads
+// stay whole: otherwise the optimizer re-partitions them along the box-sums' blocks (a row of 10
+// floats became b128 + b96 + read2_b32 + b32 instead of b128 + b128 + b64), which costs LDS
+// instructions and bank cycles. The operand is a use, so the wait for the reads stands where row_take
+// stands: behind the work that is to cover their latency, not behind the reads. The 2-float tail
+// (rather than a third float4) also keeps two registers per row free.
 typedef float lds_f4 __attribute__((ext_vector_type(4)));
 typedef float lds_f2 __attribute__((ext_vector_type(2)));
+// the vectors of such a row: NQ float4s, then one float2 if there is a tail of 1 or 2
+FL_HD constexpr int row_quads(int n) { return row_read(n) / 4; }
 template <int NV>
-__device__ __forceinline__ void lds_row(const float* __restrict__ src, float (&v)[NV]) {
-    static_assert(row_read(NV) >= NV, "row read");
+__device__ __forceinline__ void row_load(const float* __restrict__ src, lds_f4* q, lds_f2& h) {
+    static_assert(row_read(NV) >= NV && row_quads(NV) * 4 <= row_read(NV), "row read");
 #pragma unroll
-    for (int m = 0; m < NV / 4; ++m) {
-        lds_f4 f = reinterpret_cast<const lds_f4*>(src)[m];
+    for (int m = 0; m < row_quads(NV); ++m) q[m] = reinterpret_cast<const lds_f4*>(src)[m];
+    constexpr int t = row_quads(NV) * 4;
+    if constexpr (NV - t == 2) h = *reinterpret_cast<const lds_f2*>(src + t);
+    if constexpr (NV - t == 1) h.x = src[t];
+}
+template <int NV>
+__device__ __forceinline__ void row_take(const lds_f4* q, const lds_f2& h, float (&v)[NV]) {
+#pragma unroll
+    for (int m = 0; m < row_quads(NV); ++m) {
+        lds_f4 f = q[m];
         asm("" : "+v"(f));
         v[4 * m] = f.x;
         v[4 * m + 1] = f.y;
         v[4 * m + 2] = f.z;
-        v[4 * m + 3] = f.w;
+        if (4 * m + 3 < NV) v[4 * m + 3 < NV ? 4 * m + 3 : 0] = f.w;
     }
-    constexpr int t = NV / 4 * 4;
-    if constexpr (NV % 4 == 3) {
-        lds_f4 f = reinterpret_cast<const lds_f4*>(src)[NV / 4];
+    constexpr int t = row_quads(NV) * 4;
+    if constexpr (NV - t == 2) {
+        lds_f2 f = h;
         asm("" : "+v"(f));
         v[t] = f.x;
         v[t + 1] = f.y;
-        v[t + 2] = f.z;
-    } else if constexpr (NV % 4 == 2) {
-        lds_f2 f = *reinterpret_cast<const lds_f2*>(src + t);
-        asm("" : "+v"(f));
-        v[t] = f.x;
-        v[t + 1] = f.y;
-    } else if constexpr (NV % 4 == 1) {
-        float f = src[t];
+    }
+    if constexpr (NV - t == 1) {
+        float f = h.x;
         asm("" : "+v"(f));
         v[t] = f;
     }
+}
+template <int NV>
+__device__ __forceinline__ void lds_row(const float* __restrict__ src, float (&v)[NV]) {
+    lds_f4 q[row_quads(NV)];
+    lds_f2 h;
+    row_load<NV>(src, q, h);
+    row_take<NV>(q, h, v);
 }
 
 // Stores four floats to a 16-byte aligned LDS address as one 128-bit write. The vector passes
@@ -174,26 +188,39 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
     for (int j = 0; j < J; ++j) {
         int ix, iy;
         voff[j] = kOOB;
-        zaddr[j] = -1;
-        if (f_column<G>(tid + j * NT, ix, iy, zaddr[j])) {
+        // a lane past the last column repeats it (with FPAIR it writes zeros into the padding): the
+        // same values to the same address, so that no store needs a lane mask
+        const int c = G::FPAIR ? tid + j * NT : min(tid + j * NT, G::NIN - 1);
+        if (f_column<G>(c, ix, iy, zaddr[j])) {
             const int gx = x0 - 2 * HH + ix, gy = y0 - 2 * HH + iy;
             if (gx >= 0 && gx < Wd && gy >= 0 && gy < Hd) voff[j] = (uint32_t)((gy * Wd + gx) * ELEM);
         }
     }
-    if constexpr (G::FPAIR) zaddr[1] = zaddr[0] + NT;  // a lane without a second column writes padding
+    if constexpr (G::FPAIR) zaddr[1] = zaddr[0] + NT;
+    const bool f_col1 = G::FPAIR || (HH == 4 && DUAL) || wave_id * 64 + NT < G::NIN;   // this wave has second columns
     // Y items on lanes [0, YITEMS) (y-sums in P0, ncc arithmetic in P1), X and AYs units in P1,
     // AX units in P0 (lncc_geometry.h); offsets into the source and destination buffers
     // (a lane has at most one unit of X and AYs, so the two share one pair of offsets; with five
     // adjoint fields the AYs units sit on Y lanes)
-    int u_src, u_dst, a_src, a_dst, b_src, b_dst;
-    const bool has_x = x_unit<G>(tid, u_src, u_dst);
-    const bool has_a = ax_unit<G>(tid, a_src, a_dst) && ADJ;
-    const bool has_b = ays_unit<G>(tid, b_src, b_dst) && ADJ;
-    if (has_b) {
-        u_src = b_src;
-        u_dst = b_dst;
+    // The roles are whole waves (ROLE below), so that a stage is entered through one scalar compare
+    // and branch; a lane past the last unit of a role's last wave repeats that unit (the same values
+    // to the same addresses).
+    const bool wave_y = wave_id < G::NYW;
+    const bool wave_x = !wave_y && wave_id < G::NYW + G::NXW;
+    const bool wave_b = ADJ && (wave_id >= G::BL0 / 64 ? wave_id < G::BL0 / 64 + cdiv(G::BOWN, 64)
+                                                       : wave_id < cdiv(G::UB - G::BOWN, 64));
+    bool wave_a = false;
+#pragma unroll
+    for (int sl = 0; sl < G::NAW; ++sl) wave_a = wave_a || (ADJ && wave_id == ax_wave<G>(sl));
+    int u_src = 0, u_dst = 0, a_src, a_dst;
+    x_unit<G>(min(tid, G::XL0 + G::UX - 1), u_src, u_dst);
+    {
+        // the lane of the last AX unit, for the lanes past it in its wave
+        constexpr int LAST = ax_wave<G>(G::NAW - 1) * 64 + (G::UA - 1) % 64;
+        ax_unit<G>((tid >> 6) == ax_wave<G>(G::NAW - 1) ? min(tid, LAST) : tid, a_src, a_dst);
     }
-    const bool has_y = tid < G::YITEMS;
+    if (wave_b)
+        ays_unit<G>(tid >= G::BL0 ? min(tid, G::BL0 + G::BOWN - 1) : min(tid, G::UB - G::BOWN - 1), u_src, u_dst);
     int y_seg = 0, y_ax = 0;  // rows seg of AX positions
     // the Y item's offsets into Xs and Gs. At k = 7 they take the registers of the X / AYs unit
     // offsets (a Y lane has no such unit), which with three of Y's rows in flight across F is
@@ -201,12 +228,13 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
     // faster (k = 9: 1%). With both gradients the Y lanes carry AYs units, whose offsets those are.
     constexpr bool Y_SHARE = HH == 3 && !DUAL;
     int y_xs = 0, y_gs0 = 0;
-    if (has_y) {
-        y_item<G>(tid, y_seg, y_ax);
+    if (wave_y) {
+        const int item = min(tid, G::YITEMS - 1);
+        y_item<G>(item, y_seg, y_ax);
         if constexpr (Y_SHARE)
-            y_offsets<G>(tid, u_src, u_dst);
+            y_offsets<G>(item, u_src, u_dst);
         else
-            y_offsets<G>(tid, y_xs, y_gs0);
+            y_offsets<G>(item, y_xs, y_gs0);
     }
     const int y_xo = Y_SHARE ? u_src : y_xs, y_go = Y_SHARE ? u_dst : y_gs0;
     const int y_start = y_seg * G::SY;
@@ -215,8 +243,8 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
     bool y_inv[G::SY], y_core[G::SY];
     {
         const int gx = x0 - HH + y_ax;
-        const bool inx = has_y && gx >= 0 && gx < Wd;
-        const bool corex = y_ax >= HH && y_ax < HH + TX;
+        const bool inx = gx >= 0 && gx < Wd;
+        const bool corex = tid < G::YITEMS && y_ax >= HH && y_ax < HH + TX;   // a repeated item counts once
 #pragma unroll
         for (int i = 0; i < G::SY; ++i) {
             const int ay = y_start + i, gy = y0 - HH + ay;
@@ -257,8 +285,8 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
         }
     }
     {
-        const __amdgpu_buffer_rsrc_t rp = make_rsrc(pvol + (int64_t)zlo * HW * ELEM, plane_bytes);
-        const __amdgpu_buffer_rsrc_t rt = make_rsrc(tvol + (int64_t)zlo * HW * ELEM, plane_bytes);
+        const rsrc_words rp = words_at((uint64_t)(uintptr_t)pvol + (uint64_t)zlo * HW * ELEM, plane_bytes);
+        const rsrc_words rt = words_at((uint64_t)(uintptr_t)tvol + (uint64_t)zlo * HW * ELEM, plane_bytes);
 #pragma unroll
         for (int j = 0; j < J; ++j) {
             pnext[j] = load_elem<BF16>(rp, voff[j]);
@@ -279,15 +307,22 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
     const float inv_n = a.inv_n, nf = a.nf, ndr = a.ndr;
     constexpr float VS = range_scale(K);   // the range scale s = 2^-E (header)
 
-    // Plane addresses advance by one plane per step: zoff = zi * plane size, and every plane the
-    // loop touches sits at a fixed plane distance from zi. A plane outside its valid range gets a
-    // zero-sized resource (its address is never dereferenced).
+    // Plane addresses advance by one plane per step, in place: F's next plane zi+1, and AZ's output
+    // plane zo = zi-ZO with the plane after it, whose p,t are prefetched. A plane outside its valid
+    // range gets a zero-sized resource (its address is never dereferenced).
+    constexpr int ZO = 3 + 2 * HH;
     const uint64_t PB = (uint64_t)HW * ELEM;
-    const uint64_t pva = (uint64_t)(uintptr_t)pvol, tva = (uint64_t)(uintptr_t)tvol;
-    const uint64_t gva = (uint64_t)(uintptr_t)gvol, gtva = (uint64_t)(uintptr_t)gtvol;
-    uint64_t zoff = (uint64_t)zlo * PB;
+    const int64_t fz = (int64_t)(zlo + 1) * (int64_t)PB, oz = (int64_t)(zlo - ZO) * (int64_t)PB;
+    uint64_t fpa = (uint64_t)(uintptr_t)pvol + fz, fta = (uint64_t)(uintptr_t)tvol + fz;
+    uint64_t opa = (uint64_t)(uintptr_t)pvol + oz + PB, ota = (uint64_t)(uintptr_t)tvol + oz + PB;
+    uint64_t oga = (uint64_t)(uintptr_t)gvol + oz, ogta = (uint64_t)(uintptr_t)gtvol + oz;
     const int zn_hi = min(zhi, D);                 // F: new plane zi+1 valid while zi+1 < zn_hi
-    constexpr int ZO = 3 + 2 * HH;                 // AZ: output plane zi-ZO
+    // Stage ranges: X(zi) runs for t = zi - HH - zc_lo in [0, nz), Y one step later, AX and AYs two,
+    // AZ's input three: one subtraction and one unsigned compare each, zero planes for a wave
+    // without the role.
+    const int tb = HH + zc_lo;
+    const uint32_t nz = (uint32_t)(zc_hi - zc_lo);
+    const uint32_t n_x = wave_x ? nz : 0u, n_y = wave_y ? nz : 0u, n_a = wave_a ? nz : 0u, n_b = wave_b ? nz : 0u;
     // z-window chains (zstep5 / zstep1): the previous block's sums over ring slots F_CHAIN..K-1
     // (F) and A_CHAIN..K-1 (AZ) kept as partial sums; 0 = none. F's chain (slots 4..6 at k = 7)
     // saves adds but holds five more registers per column; at k = 7 those registers measured
@@ -319,7 +354,7 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
             const float ncc = (X * VS) * cr;     // ncc
             const bool live = y_inv[i] && (ncc < 1.0f);
             const float nccc = (ncc >= 1.0f) ? 1.0f : ncc;
-            if (count && y_core[i]) lsum += nccc;
+            if (y_core[i]) lsum += nccc;
             if constexpr (ADJ) {
                 // masking cr masks all three coefficients (alpha, beta, gamma are multiples of it)
                 const float crm = live ? cr : 0.f;
@@ -360,7 +395,7 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
             for (int c = 0; c < NADJ; ++c)
                 lds_store4(Gs + y_go + c * G::GP, adj[c][0], adj[c][1], adj[c][2], adj[c][3]);
         }
-        loss_acc += (double)lsum;
+        if (count) loss_acc += (double)lsum;
     };
     // F(zi): z-sums of the input region over planes [zi-k+1, zi] (zstep5: the plane prefetched one
     // step ago joins the block prefix and the ring, the previous block's suffix comes from the
@@ -374,88 +409,86 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
         constexpr bool STORE = decltype(store)::value;
 #pragma unroll
         for (int j = decltype(jb)::value; j < decltype(je)::value; ++j) {
+            if (j > 0 && !f_col1) continue;
             zstep5<K, r, F_CHAIN>(pnext[j], tnext[j], fpre[j], pring[j], tring[j], fch[j], zsum[j]);
             if constexpr (STORE) {
-                if (G::FPAIR || zaddr[j] >= 0) {
-#pragma unroll
-                    for (int q = 0; q < 5; ++q) Zs[q * G::ZP + zaddr[j]] = zsum[j][q];
-                }
-            }
-        }
-    };
-    auto f_pref = [&](int zi, uint64_t zoff) __attribute__((always_inline)) {
-        // prefetch plane zi+1
-        const bool okn = zi + 1 < zn_hi;
-        const __amdgpu_buffer_rsrc_t rpn = rsrc_at(pva + zoff + PB, plane_bytes, okn);
-        const __amdgpu_buffer_rsrc_t rtn = rsrc_at(tva + zoff + PB, plane_bytes, okn);
-#pragma unroll
-        for (int j = 0; j < J; ++j) {
-            pnext[j] = load_elem<BF16>(rpn, voff[j]);
-            tnext[j] = load_elem<BF16>(rtn, voff[j]);
-        }
-    };
-    auto f_sums = [&](auto rc, auto store, int zi, uint64_t zoff) __attribute__((always_inline)) {
-        f_cols(rc, store, std::integral_constant<int, 0>{}, std::integral_constant<int, J>{});
-        f_pref(zi, zoff);
-    };
-    auto f_store = [&]() __attribute__((always_inline)) {
-#pragma unroll
-        for (int j = 0; j < J; ++j) {
-            if (zaddr[j] >= 0) {
 #pragma unroll
                 for (int q = 0; q < 5; ++q) Zs[q * G::ZP + zaddr[j]] = zsum[j][q];
             }
         }
     };
+    auto f_pref = [&](int zi) __attribute__((always_inline)) {
+        // prefetch plane zi+1
+        const uint32_t nb = zi + 1 < zn_hi ? plane_bytes : 0u;
+        const rsrc_words rpn = words_at(fpa, nb), rtn = words_at(fta, nb);
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            pnext[j] = load_elem<BF16>(rpn, voff[j]);
+            tnext[j] = load_elem<BF16>(rtn, voff[j]);
+        }
+        fpa += PB;
+        fta += PB;
+    };
+    auto f_sums = [&](auto rc, auto store, int zi) __attribute__((always_inline)) {
+        f_cols(rc, store, std::integral_constant<int, 0>{}, std::integral_constant<int, J>{});
+        f_pref(zi);
+    };
+    auto f_store = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            if (j > 0 && !f_col1) continue;
+#pragma unroll
+            for (int q = 0; q < 5; ++q) Zs[q * G::ZP + zaddr[j]] = zsum[j][q];
+        }
+    };
     // Stage order inside a phase. Each wave runs its stages in program order, so a stage placed
     // between the issue of another stage's LDS reads and their use hides part of their latency.
-    //  * P0: AZ's xy-sums are read first. The Y lanes read Y_EARLY of their five rows (all five
-    //    at k <= 5, three at k = 7, two for bf16 at k = 7: more rows held across F exceed the
-    //    128-register budget of a 1024-lane workgroup) and at k <= 5 the AX lanes their row; F
-    //    runs while they arrive, then the Y lanes read their other rows and form the five box
-    //    sums, which stay in registers until P1, and the AX lanes their sums; AZ's z-sums and the
-    //    gradient come last. At k = 9 (two rings of 9 planes) nothing is read before F, one row
-    //    between F's two columns, and the others one at a time after F. (At k = 7 the AX row read
-    //    before F measured 1% slower than after it.)
+    //  * P0: AZ's xy-sums are read first. The Y waves issue the reads of Y_EARLY of their five rows
+    //    (with the adjoint five at k = 3, three at k = 5, two at k = 7, none at k = 9: more rows held
+    //    across F exceed the 128-register budget of a 1024-lane workgroup) and at k <= 5 the AX waves
+    //    those of their row; F runs while they arrive (the wait stands at row_take), then the Y waves
+    //    read their other rows and form the five box sums, which stay in registers until P1, and the
+    //    AX waves their sums; AZ's z-sums and the gradient come last.
     //  * P1: the Y lanes turn their box sums into ncc and the adjoint coefficients (arithmetic
     //    only, no LDS reads: it keeps the SIMDs busy while the rows of the X and AYs units, on the
     //    other waves, arrive), then the X and AYs units (with both gradients, at k >= 5, also on
     //    the first Y lanes: units that do not fit after the X units, 2-7% faster than all AYs
     //    units on Y lanes).
     //  * Both gradients (five adjoint fields, fourteen more ring registers per lane at k = 7):
-    //    fewer early rows, all five at k = 3, two (bf16) or none (fp32) at k = 5, one at k = 7
-    //    (more early rows spill; the counts are the fastest measured: k = 5 fp32 with none 1.2% faster than with
-    //    two, bf16 with two 0.4% faster than with none), and no AX row before F. At k = 9 the two
-    //    9-plane rings and the five adjoint rings exceed the 128 registers even so: 36-46 spill to
-    //    scratch, and the launch still runs 22-26% faster than two pred-gradient passes.
-    constexpr int Y_EARLY = DUAL ? (HH <= 1 ? 5 : HH == 2 ? (BF16 ? 2 : 0) : HH == 3 ? 1 : 0)
-                                 : HH <= 2 ? 5 : HH == 3 ? (BF16 ? 2 : 3) : 0;   // Y rows read before F
+    //    fewer early rows, all five at k = 3, two (bf16) or none (fp32) at k = 5, none above, and no
+    //    AX row before F. At k = 9 the two 9-plane rings and the five adjoint rings exceed the 128
+    //    registers even so: 36-54 spill to scratch, and the launch still runs a quarter faster than
+    //    two pred-gradient passes.
+    // What a step costs: 16 waves, 4 per SIMD, none of VALU issue (~55% of the step), LDS (58% active)
+    // or HBM (25%) saturated. A scalar instruction takes an issue cycle of its wave like a vector one,
+    // and a step had 92 of them for 149 vector ones: lane masks for roles that are whole waves, and
+    // five buffer resources rebuilt from 64-bit addresses. Roles as scalar branches and addresses
+    // advanced in place leave about 55; with the row waits moved behind F, (2,16,128^3) went from
+    // 0.344 / 0.369 / 0.401 / 0.584 to 0.331 / 0.359 / 0.391 / 0.564 ms at k = 3 / 5 / 7 / 9.
+    constexpr int Y_EARLY = DUAL ? (HH <= 1 ? 5 : HH == 2 ? (BF16 ? 2 : 0) : 0)
+                                 : !ADJ ? (HH <= 2 ? 5 : HH == 3 ? 3 : 0)
+                                 : HH <= 1 ? 5 : HH == 2 ? 3 : HH == 3 ? 2 : 0;   // Y rows read before F
     constexpr bool F_STORE_AT_ONCE = Y_EARLY < 5;
     // Y_MID of Y's rows are read between F's two columns, after the box sums of the early rows
-    // (whose registers they take); the rest after F. k = 9: one row (0.6-1% faster than none).
-    // k = 7: one row measured 0.7% faster at (2,16,128^3) but 1.3% slower at (2,16,256^3), whose
-    // re-reads of the output planes then missed the L2 more often (HBM reads 1.05x -> up to 1.46x
-    // the inputs, growing from launch to launch); none.
-    constexpr int Y_MID = HH == 4 && J == 2 && !DUAL ? 1 : 0;
+    // (whose registers they take); the rest after F. k = 9 without the adjoint: one row; with it, none
+    // (the row spills registers, 3% slower).
+    constexpr int Y_MID = HH == 4 && J == 2 && !ADJ ? 1 : 0;
     static_assert(Y_EARLY + Y_MID <= 5, "Y rows");
     constexpr bool AX_EARLY = HH <= 2 && !DUAL;               // the AX row read before F
     constexpr int NY = G::SY + 2 * HH, NA = G::SA + 2 * HH, NX = G::SX + 2 * HH, NB = G::SB + 2 * HH;
     // P0's early reads (Y's first rows or the AX row) share one register array: the two kinds of
     // lane sit on different waves
-    constexpr int NE0 = cmax(cmax(Y_EARLY * NY, AX_EARLY ? NA : 0), NY);
+    constexpr int YQ = row_quads(NY);
+    constexpr int NEQ = cmax(cmax(Y_EARLY * YQ, AX_EARLY ? row_quads(NA) : 0), 1), NEH = cmax(Y_EARLY, 1);
 
     for (int base = zlo; base < zhi; base += K) {
         static_for<0, K>([&](auto rc) __attribute__((always_inline)) {
             const int zi = base + decltype(rc)::value;
             if (zi >= zhi) return;
-            const int zcX = zi - HH;       // X(zi): the z-sums of F(zi) are centred on plane zi-h
-            const bool actX = zcX >= zc_lo && zcX < zc_hi;
-            const int zcY = zi - 1 - HH;   // Y(zi-1)
-            const bool actY = zcY >= zc_lo && zcY < zc_hi;
-            const int zcB = zi - 2 - HH;   // AX(zi-2) and AYs(zi-2)
-            const bool actB = ADJ && zcB >= zc_lo && zcB < zc_hi;
-            const int zcA = zi - 3 - HH;   // the xy-sums AZ(zi-3) reads
-            const bool actA = ADJ && zcA >= zc_lo && zcA < zc_hi;
+            const int zcY = zi - 1 - HH;   // the plane Y(zi-1) is centred on (the z-sums of F(z): z-h)
+            const uint32_t t = (uint32_t)(zi - tb);
+            const bool do_x = t < n_x, do_y = t - 1u < n_y, do_a = t - 2u < n_a, do_b = t - 2u < n_b;
+            const bool actA = ADJ && t - 3u < nz;   // the xy-sums AZ(zi-3) reads
 
             // ============================ phase P0 ============================
             // AZ(zi-3) reads, Y(zi-1) y-sums, AX(zi-2), F(zi), AZ(zi-3)
@@ -471,70 +504,56 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
                 }
             };
             if constexpr (ADJ && HH <= 3) az_read();
-            float er[NE0];
-            if (has_y && actY) {
+            lds_f4 eq[NEQ];
+            lds_f2 eh[NEH];
+            if (do_y) {
 #pragma unroll
-                for (int q = 0; q < Y_EARLY; ++q) {
-                    float v[NY];
-                    lds_row(Xs + q * G::XP + y_xo, v);
-#pragma unroll
-                    for (int i = 0; i < NY; ++i) er[q * NY + i] = v[i];
-                }
-            } else if (AX_EARLY && has_a && actB) {
-                float v[NA];
-                lds_row(Gs + a_src, v);
-#pragma unroll
-                for (int i = 0; i < NA; ++i) er[i] = v[i];
+                for (int q = 0; q < Y_EARLY; ++q) row_load<NY>(Xs + q * G::XP + y_xo, eq + q * YQ, eh[q]);
+            } else if (AX_EARLY && do_a) {
+                row_load<NA>(Gs + a_src, eq, eh[0]);
             }
             float S[5][G::SY];  // Y's box sums, carried into P1
-            float em[Y_MID > 0 ? Y_MID * NY : 1];
+            lds_f4 mq[cmax(Y_MID * YQ, 1)];
+            lds_f2 mh[cmax(Y_MID, 1)];
             if constexpr (Y_MID > 0) {
                 // F's first column; then the box sums of the early rows and the reads of the mid
                 // rows; then F's second column and the prefetch
                 f_cols(rc, std::true_type{}, std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{});
-                if (has_y && actY) {
+                if (do_y) {
 #pragma unroll
                     for (int q = 0; q < Y_EARLY; ++q) {
                         float v[NY];
-#pragma unroll
-                        for (int i = 0; i < NY; ++i) v[i] = er[q * NY + i];
+                        row_take<NY>(eq + q * YQ, eh[q], v);
                         box_sums<HH, G::SY>(v, S[q]);
                     }
 #pragma unroll
-                    for (int q = 0; q < Y_MID; ++q) {
-                        float v[NY];
-                        lds_row(Xs + (Y_EARLY + q) * G::XP + y_xo, v);
-#pragma unroll
-                        for (int i = 0; i < NY; ++i) em[q * NY + i] = v[i];
-                    }
+                    for (int q = 0; q < Y_MID; ++q)
+                        row_load<NY>(Xs + (Y_EARLY + q) * G::XP + y_xo, mq + q * YQ, mh[q]);
                 }
                 f_cols(rc, std::true_type{}, std::integral_constant<int, 1>{}, std::integral_constant<int, J>{});
-                f_pref(zi, zoff);
+                f_pref(zi);
             } else {
-                f_sums(rc, std::integral_constant<bool, F_STORE_AT_ONCE>{}, zi, zoff);
+                f_sums(rc, std::integral_constant<bool, F_STORE_AT_ONCE>{}, zi);
             }
-            if (has_y && actY) {
+            if (do_y) {
                 // the rows not yet summed: early rows (held in er), mid rows (em), the rest read now
 #pragma unroll
                 for (int q = Y_MID > 0 ? Y_EARLY : 0; q < 5; ++q) {
                     float v[NY];
                     if (q < Y_EARLY) {
-#pragma unroll
-                        for (int i = 0; i < NY; ++i) v[i] = er[(q < Y_EARLY ? q : 0) * NY + i];
+                        row_take<NY>(eq + q * YQ, eh[q < Y_EARLY ? q : 0], v);
                     } else if (q < Y_EARLY + Y_MID) {
-#pragma unroll
-                        for (int i = 0; i < NY; ++i) v[i] = em[(q < Y_EARLY + Y_MID ? q - Y_EARLY : 0) * NY + i];
+                        row_take<NY>(mq + (q - Y_EARLY) * YQ, mh[q < Y_EARLY + Y_MID ? q - Y_EARLY : 0], v);
                     } else {
                         lds_row(Xs + q * G::XP + y_xo, v);
                     }
                     box_sums<HH, G::SY>(v, S[q]);
                 }
-            } else if (has_a && actB) {
+            } else if (do_a) {
                 // AX(zi-2): x-sums (y-sums with ASWAP) of one of alpha, beta, gamma over one segment
                 float v[NA], o[G::SA];
                 if constexpr (AX_EARLY) {
-#pragma unroll
-                    for (int i = 0; i < NA; ++i) v[i] = er[i];
+                    row_take<NA>(eq, eh[0], v);
                 } else {
                     lds_row(Gs + a_src, v);
                 }
@@ -563,30 +582,35 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
                 // tile are half a 128-byte line (the x-neighbour tile writes the other half):
                 // those stores keep the default policy, so that the L2 merges the two halves into
                 // one write.
-                store_elem_buf<BF16, BF16 ? 0 : kNT>(rsrc_at(gva + zoff - ZO * PB, plane_bytes, zo >= z0 && zo < z1), z_voff, g);
+                const uint32_t gb = zo >= z0 ? plane_bytes : 0u;   // zo < z1 up to the march's last step
+                store_elem_buf<BF16, BF16 ? 0 : kNT>(words_at(oga, gb), z_voff, g);
+                oga += PB;
                 if constexpr (DUAL) {
                     const float gt = a.gscale * fmaf(inv_n, gw[3], fmaf(tzz, gw[4], -pz * gw[2]));
-                    store_elem_buf<BF16, BF16 ? 0 : kNT>(rsrc_at(gtva + zoff - ZO * PB, plane_bytes, zo >= z0 && zo < z1), z_voff, gt);
+                    store_elem_buf<BF16, BF16 ? 0 : kNT>(words_at(ogta, gb), z_voff, gt);
+                    ogta += PB;
                 }
                 // prefetch p,t at the next step's output plane; issued after this step's use, so
                 // one register each suffices and no copy has to wait for the load
-                const bool oko = zo + 1 >= z0 && zo + 1 < z1;
-                pz = load_elem<BF16, kNT>(rsrc_at(pva + zoff - (ZO - 1) * PB, plane_bytes, oko), z_voff);
-                tzz = load_elem<BF16, kNT>(rsrc_at(tva + zoff - (ZO - 1) * PB, plane_bytes, oko), z_voff);
+                const uint32_t ob = (uint32_t)(zo + 1 - z0) < (uint32_t)(z1 - z0) ? plane_bytes : 0u;
+                pz = load_elem<BF16, kNT>(words_at(opa, ob), z_voff);
+                tzz = load_elem<BF16, kNT>(words_at(ota, ob), z_voff);
+                opa += PB;
+                ota += PB;
             }
             __syncthreads();
 
             // ============================ phase P1 ============================
             // Y(zi-1) ncc arithmetic, X(zi), AYs(zi-2)
-            if (has_y && actY) y_math(S, zcY);
-            if (has_x && actX) {
+            if (do_y) y_math(S, zcY);
+            if (do_x) {
                 // X(zi): x-sums of one of the five z-sums over one segment (feeds Y at the next plane)
                 float v[NX], o[G::SX];
                 lds_row(Zs + u_src, v);
                 box_sums<HH, G::SX>(v, o);
 #pragma unroll
                 for (int i = 0; i < G::SX; ++i) Xs[u_dst + i * G::XS] = o[i];
-            } else if (has_b && actB) {
+            } else if (do_b) {
                 // AYs(zi-2): y-sums (x-sums with ASWAP) of one of alpha, beta, gamma at plane zcB
                 float v[NB], o[G::SB];
                 lds_row(GXs + u_src, v);
@@ -601,7 +625,6 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
                     }
                 }
             }
-            zoff += PB;
             __syncthreads();
         });
     }

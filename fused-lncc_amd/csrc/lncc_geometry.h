@@ -93,7 +93,7 @@ struct Geo {
     // not fit on the lanes after the X units (BOWN of them do) run on the first Y lanes, after Y's
     // ncc arithmetic (which reads no LDS row).
     static constexpr int UX = 5 * XITEMS, UA = NA * AITEMS, UB = NA * BITEMS;
-    static constexpr int NYW = cdiv(YITEMS, 64), XL0 = 64 * NYW, BL0 = rup64(XL0 + UX), NAW = cdiv(UA, 64);
+    static constexpr int NYW = cdiv(YITEMS, 64), XL0 = 64 * NYW, NXW = cdiv(UX, 64), BL0 = rup64(XL0 + UX), NAW = cdiv(UA, 64);
     static constexpr int BOWN = UB < NT - BL0 ? UB : NT - BL0;
     static constexpr bool B_ON_Y = UB > BOWN;
     // Y items and X units on disjoint lanes, AYs units on lanes of their own or on Y lanes (the
