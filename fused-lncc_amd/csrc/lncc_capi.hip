@@ -3,6 +3,7 @@
 #include <stdio.h>
 #include <stdlib.h>
 
+#include <algorithm>
 #include <atomic>
 #include <string>
 
@@ -92,6 +93,50 @@ Plan plan_fused(int64_t B, int64_t D, int64_t H, int64_t W, int halo) {
     return p;
 }
 
+// The forward-only kernel's launch (the loss without a gradient, the maps): tiles of 16 * cols
+// columns, nzc chunks of dchunk planes per tile, taken in turn by nblocks workgroups.
+struct ForwardPlan {
+    int cols, ntx, nty, nzc, dchunk;
+    int64_t npieces, nblocks;
+};
+
+// The best split of tiles of one width, if better than `best`: a chunk of d planes costs d + 2h + 1
+// planes of cost `step`, and the workgroups, one per CU, take the chunks in rounds. Never more
+// workgroups than the gradient plan's `gblocks`, whose count the reduction of the partial sums reads.
+template <int H, int NC>
+void try_forward(int64_t B, int64_t D, int64_t H_, int64_t W, int64_t gblocks, double step, ForwardPlan& f, double& best) {
+    using G = fl::FwdGeo<H, NC>;
+    const int64_t ntx = W <= G::RW ? 1 : 1 + (W - G::RW + G::ADV - 1) / G::ADV, nty = (H_ + G::OY - 1) / G::OY;
+    const int64_t tiles = B * ntx * nty, most = std::min<int64_t>(device_cus(), gblocks);
+    for (int64_t nzc = 1; nzc <= D; ++nzc) {
+        const int64_t d = t_dchunk_override > 0 ? std::min(t_dchunk_override, D) : (D + nzc - 1) / nzc;
+        const int64_t n = (D + d - 1) / d, pieces = tiles * n;
+        const double cost = (double)((pieces + most - 1) / most) * (double)(d + 2 * H + 1) * step;
+        if (best < 0 || cost < best) {
+            best = cost;
+            f = ForwardPlan{NC, (int)ntx, (int)nty, (int)n, (int)d, pieces, std::min(pieces, most)};
+        }
+        if (pieces >= 4 * most || t_dchunk_override > 0) break;
+    }
+}
+
+ForwardPlan plan_forward(int64_t B, int64_t D, int64_t H, int64_t W, int halo, bool maps, int64_t gblocks) {
+    ForwardPlan f = {};
+    double best = -1;
+    // A plane of a 64-column tile (28 output rows) against one of a 48-column tile (32): 1.1x measured at
+    // k <= 5; at k = 7, where the four columns' rings fill the registers and a few spill, 1.13x for the
+    // loss ((2,64,64^3): 109 us in 64-column tiles, 117 in 48-column ones) and 1.4x for the maps
+    // (160x192x224: 38-41 and 34 us). At k = 9 they don't fit.
+    const double wide7 = maps ? 1.4 : 1.2;
+    switch (halo) {
+        case 1: try_forward<1, 3>(B, D, H, W, gblocks, 1.0, f, best); try_forward<1, 4>(B, D, H, W, gblocks, 1.1, f, best); break;
+        case 2: try_forward<2, 3>(B, D, H, W, gblocks, 1.0, f, best); try_forward<2, 4>(B, D, H, W, gblocks, 1.1, f, best); break;
+        case 3: try_forward<3, 3>(B, D, H, W, gblocks, 1.0, f, best); try_forward<3, 4>(B, D, H, W, gblocks, wide7, f, best); break;
+        default: try_forward<4, 3>(B, D, H, W, gblocks, 1.0, f, best); break;
+    }
+    return f;
+}
+
 // A launch of n workgroups of `lanes` lanes: the grid in lanes must fit in 32 bits.
 bool grid_fits(int64_t n, int lanes) { return n >= 1 && n <= (int64_t)0xffffffffLL / lanes; }
 
@@ -149,6 +194,20 @@ hipError_t launch_fused(int halo, int mode, bool bf16, const fl::FusedArgs& a, c
         case 4: return fl::launch_fused_h4(mode, bf16, a, nb, st);
         default: return hipErrorInvalidValue;
     }
+}
+
+// The loss without a gradient, or the maps. `a` holds the arguments of the gradient plan g.
+hipError_t launch_forward(int64_t B, int halo, int mode, bool bf16, fl::FusedArgs a, const Plan& g, hipStream_t st) {
+    if (g.small) return fl::launch_small(halo, mode, bf16, a, (uint32_t)g.nblocks, st);
+    const ForwardPlan f = plan_forward(B, a.dimD, a.dimH, a.dimW, halo, mode == fl::MODE_MAPS, g.nblocks);
+    a.ntx = f.ntx;
+    a.nty = f.nty;
+    a.nzc = f.nzc;
+    a.dchunk = f.dchunk;
+    a.nparts = (uint32_t)g.nblocks;
+    if (f.npieces > 0xffffffffLL - f.nblocks) return hipErrorInvalidValue;   // a tile count that fits a grid is far below
+    a.npieces = (uint32_t)f.npieces;
+    return fl::launch_forward(halo, f.cols, mode, bf16, a, (uint32_t)f.nblocks, st);
 }
 
 // Kernel arguments shared by every mode of the fused kernel; mode-specific outputs are set by the
@@ -280,8 +339,9 @@ int fl_lncc_fused_partials(const void* pred, const void* target, int dtype, int6
     fl::FusedArgs a = fused_args(pred, target, B, D, H, W, kernel_size, smooth_dr, p);
     a.grad = grad;
     a.partials = static_cast<double*>(workspace);
-    hipError_t e = launch_fused(halo, grad ? fl::MODE_GRAD : fl::MODE_LOSS, dtype == FL_BF16, a, p,
-                                static_cast<hipStream_t>(stream));
+    const hipStream_t st = static_cast<hipStream_t>(stream);
+    hipError_t e = grad ? launch_fused(halo, fl::MODE_GRAD, dtype == FL_BF16, a, p, st)
+                        : launch_forward(B, halo, fl::MODE_LOSS, dtype == FL_BF16, a, p, st);
     if (e != hipSuccess) return hip_fail(e, "fl_lncc_fused_partials: fused kernel launch");
     return FL_OK;
 }
@@ -336,7 +396,8 @@ int fl_lncc_loss_grad_noalloc(const void* pred, const void* target, int dtype, i
     a.grad = grad;
     a.partials = part;
     const hipStream_t st = static_cast<hipStream_t>(stream);
-    hipError_t e = launch_fused(halo, grad ? fl::MODE_GRAD : fl::MODE_LOSS, dtype == FL_BF16, a, p, st);
+    hipError_t e = grad ? launch_fused(halo, fl::MODE_GRAD, dtype == FL_BF16, a, p, st)
+                        : launch_forward(B, halo, fl::MODE_LOSS, dtype == FL_BF16, a, p, st);
     if (e != hipSuccess) return hip_fail(e, "fl_lncc_loss_grad_noalloc: fused kernel launch");
     const double M = (double)B * (double)D * (double)H * (double)W;
     e = fl::launch_finalize(part, (int)p.nblocks, 1.0 / M, loss, st);
@@ -404,8 +465,7 @@ int fl_lncc_maps(const void* pred, const void* target, int dtype, int64_t B, int
     a.a_map = A;
     a.b_map = Bc;
     a.c_map = Cc;
-    hipError_t e = launch_fused(halo, fl::MODE_MAPS, dtype == FL_BF16, a, p,
-                                static_cast<hipStream_t>(stream));
+    hipError_t e = launch_forward(B, halo, fl::MODE_MAPS, dtype == FL_BF16, a, p, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, "fl_lncc_maps: launch");
     return FL_OK;
 }

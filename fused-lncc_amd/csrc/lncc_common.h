@@ -29,6 +29,10 @@ __device__ __forceinline__ rsrc_words words_at(uint64_t addr, uint32_t bytes) {
     return rsrc_words{(int)(uint32_t)addr, (int)(uint32_t)(addr >> 32), (int)bytes, kRsrcWord3};
 }
 __device__ float raw_load_f32(rsrc_words r, int voff, int soff, int aux) __asm("llvm.amdgcn.raw.buffer.load.f32");
+typedef float f32x3 __attribute__((ext_vector_type(3)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+__device__ f32x3 raw_load_f32x3(rsrc_words r, int voff, int soff, int aux) __asm("llvm.amdgcn.raw.buffer.load.v3f32");
+__device__ f32x4 raw_load_f32x4(rsrc_words r, int voff, int soff, int aux) __asm("llvm.amdgcn.raw.buffer.load.v4f32");
 __device__ unsigned short raw_load_b16(rsrc_words r, int voff, int soff, int aux) __asm("llvm.amdgcn.raw.buffer.load.i16");
 __device__ void raw_store_f32(float v, rsrc_words r, int voff, int soff, int aux) __asm("llvm.amdgcn.raw.buffer.store.f32");
 __device__ void raw_store_b16(unsigned short v, rsrc_words r, int voff, int soff, int aux) __asm("llvm.amdgcn.raw.buffer.store.i16");
@@ -55,6 +59,19 @@ __device__ __forceinline__ float load_elem(rsrc_words r, uint32_t voff) {
         return __uint_as_float((uint32_t)raw_load_b16(r, (int)voff, 0, AUX) << 16);
     else
         return raw_load_f32(r, (int)voff, 0, AUX);
+}
+
+// N = 3 or 4 consecutive floats in one load (4-byte aligned)
+template <int N>
+__device__ __forceinline__ void load_run(rsrc_words r, uint32_t voff, float (&v)[N]) {
+    static_assert(N == 3 || N == 4, "runs");
+    if constexpr (N == 3) {
+        const f32x3 f = raw_load_f32x3(r, (int)voff, 0, 0);
+        v[0] = f.x, v[1] = f.y, v[2] = f.z;
+    } else {
+        const f32x4 f = raw_load_f32x4(r, (int)voff, 0, 0);
+        v[0] = f.x, v[1] = f.y, v[2] = f.z, v[3] = f.w;
+    }
 }
 
 template <bool BF16>

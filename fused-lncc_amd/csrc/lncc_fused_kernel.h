@@ -1,4 +1,4 @@
-// Fused 3D LNCC kernels for gfx950 (MI355X).
+// Fused 3D LNCC kernel for gfx950 (MI355X): the loss and the pred gradient, or both gradients.
 //
 // One workgroup (1024 lanes) owns a TX x TY tile of output columns of one (D,H,W) volume and
 // marches along D over a chunk [z0,z1) of planes. Per input plane zi it runs six stages, lagged
@@ -64,79 +64,15 @@
 #pragma once
 #include "lncc_common.h"
 #include "lncc_launch.h"
+#include "lncc_lds.h"
 #include "lncc_window.h"
 
 namespace fl {
 
-// A row of NV consecutive floats at a 16-byte aligned LDS address, read as float4s, then a tail of 2
-// or 1 floats as a float2 or a float (a tail of 3 as one more float4, which reads one float past the
-// row; it is not used), row_read(NV) floats in all. row_load issues the reads; row_take hands out the
-// values, each vector through an empty asm operand that needs all of its lanes, so that the loads
-// stay whole: otherwise the optimizer re-partitions them along the box-sums' blocks (a row of 10
-// floats became b128 + b96 + read2_b32 + b32 instead of b128 + b128 + b64), which costs LDS
-// instructions and bank cycles. The operand is a use, so the wait for the reads stands where row_take
-// stands: behind the work that is to cover their latency, not behind the reads. The 2-float tail
-// (rather than a third float4) also keeps two registers per row free.
-typedef float lds_f4 __attribute__((ext_vector_type(4)));
-typedef float lds_f2 __attribute__((ext_vector_type(2)));
-// the vectors of such a row: NQ float4s, then one float2 if there is a tail of 1 or 2
-FL_HD constexpr int row_quads(int n) { return row_read(n) / 4; }
-template <int NV>
-__device__ __forceinline__ void row_load(const float* __restrict__ src, lds_f4* q, lds_f2& h) {
-    static_assert(row_read(NV) >= NV && row_quads(NV) * 4 <= row_read(NV), "row read");
-#pragma unroll
-    for (int m = 0; m < row_quads(NV); ++m) q[m] = reinterpret_cast<const lds_f4*>(src)[m];
-    constexpr int t = row_quads(NV) * 4;
-    if constexpr (NV - t == 2) h = *reinterpret_cast<const lds_f2*>(src + t);
-    if constexpr (NV - t == 1) h.x = src[t];
-}
-template <int NV>
-__device__ __forceinline__ void row_take(const lds_f4* q, const lds_f2& h, float (&v)[NV]) {
-#pragma unroll
-    for (int m = 0; m < row_quads(NV); ++m) {
-        lds_f4 f = q[m];
-        asm("" : "+v"(f));
-        v[4 * m] = f.x;
-        v[4 * m + 1] = f.y;
-        v[4 * m + 2] = f.z;
-        if (4 * m + 3 < NV) v[4 * m + 3 < NV ? 4 * m + 3 : 0] = f.w;
-    }
-    constexpr int t = row_quads(NV) * 4;
-    if constexpr (NV - t == 2) {
-        lds_f2 f = h;
-        asm("" : "+v"(f));
-        v[t] = f.x;
-        v[t + 1] = f.y;
-    }
-    if constexpr (NV - t == 1) {
-        float f = h.x;
-        asm("" : "+v"(f));
-        v[t] = f;
-    }
-}
-template <int NV>
-__device__ __forceinline__ void lds_row(const float* __restrict__ src, float (&v)[NV]) {
-    lds_f4 q[row_quads(NV)];
-    lds_f2 h;
-    row_load<NV>(src, q, h);
-    row_take<NV>(q, h, v);
-}
-
-// Stores four floats to a 16-byte aligned LDS address as one 128-bit write. The vector passes
-// through an empty asm operand that needs all of its lanes, for the reason given at lds_row: left
-// alone, the compiler split the AYs stores into pairs of adjacent 32-bit writes (ds_write2_b32),
-// and at the row stride of GY (36 floats) each such write served 64 lanes from 16 banks, 4-way
-// conflicts: a quarter of the kernel's LDS bank-conflict cycles came from them.
-__device__ __forceinline__ void lds_store4(float* __restrict__ dst, float x, float y, float z, float w) {
-    lds_f4 f = {x, y, z, w};
-    asm("" : "+v"(f));
-    *reinterpret_cast<lds_f4*>(dst) = f;
-}
-
 template <int HH, bool BF16, int MODE>
 __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) {
     constexpr bool DUAL = (MODE == MODE_DUAL);
-    constexpr bool ADJ = (MODE == MODE_GRAD) || DUAL;
+    static_assert(MODE == MODE_GRAD || DUAL, "the loss alone and the maps: lncc_forward_kernel.h");
     constexpr int NADJ = DUAL ? 5 : 3;   // adjoint fields
     using G = Geo<HH, NADJ>;
     constexpr int K = G::K;
@@ -148,9 +84,9 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
     // alias the writes of another and can overlap them
     __shared__ __align__(16) float Zs[5 * G::ZP + G::PAD];
     __shared__ __align__(16) float Xs[5 * G::XP + G::PAD];
-    __shared__ __align__(16) float Gs[ADJ ? NADJ * G::GP + G::PAD : 4];
-    __shared__ __align__(16) float GXs[ADJ ? NADJ * G::GXP + G::PAD : 4];
-    __shared__ __align__(16) float GY[ADJ ? NADJ * G::GYP : 2];
+    __shared__ __align__(16) float Gs[NADJ * G::GP + G::PAD];
+    __shared__ __align__(16) float GXs[NADJ * G::GXP + G::PAD];
+    __shared__ __align__(16) float GY[NADJ * G::GYP];
     __shared__ double red[NT / 64];
 
     const int tid = threadIdx.x;
@@ -178,7 +114,7 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
     const uint32_t plane_bytes = (uint32_t)(HW * ELEM);
     const char* pvol = (const char*)a.pred + b * D * HW * ELEM;
     const char* tvol = (const char*)a.target + b * D * HW * ELEM;
-    char* const gvol = ADJ ? (char*)a.grad + b * D * HW * ELEM : nullptr;
+    char* const gvol = (char*)a.grad + b * D * HW * ELEM;
     char* const gtvol = DUAL ? (char*)a.grad_t + b * D * HW * ELEM : nullptr;
 
     // ---- F: per-lane input columns
@@ -207,11 +143,11 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
     // to the same addresses).
     const bool wave_y = wave_id < G::NYW;
     const bool wave_x = !wave_y && wave_id < G::NYW + G::NXW;
-    const bool wave_b = ADJ && (wave_id >= G::BL0 / 64 ? wave_id < G::BL0 / 64 + cdiv(G::BOWN, 64)
-                                                       : wave_id < cdiv(G::UB - G::BOWN, 64));
+    const bool wave_b = wave_id >= G::BL0 / 64 ? wave_id < G::BL0 / 64 + cdiv(G::BOWN, 64)
+                                               : wave_id < cdiv(G::UB - G::BOWN, 64);
     bool wave_a = false;
 #pragma unroll
-    for (int sl = 0; sl < G::NAW; ++sl) wave_a = wave_a || (ADJ && wave_id == ax_wave<G>(sl));
+    for (int sl = 0; sl < G::NAW; ++sl) wave_a = wave_a || wave_id == ax_wave<G>(sl);
     int u_src = 0, u_dst = 0, a_src, a_dst;
     x_unit<G>(min(tid, G::XL0 + G::UX - 1), u_src, u_dst);
     {
@@ -252,17 +188,16 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
             y_core[i] = y_inv[i] && corex && ay >= HH && ay < HH + TY;
         }
     }
-    const bool has_z = ADJ && tid < G::NOUT;
+    const bool has_z = tid < G::NOUT;
     int z_ox, z_oy;
     az_lane<G>(tid, z_ox, z_oy);
     const bool z_in = has_z && x0 + z_ox < Wd && y0 + z_oy < Hd;
     const uint32_t z_voff = z_in ? (uint32_t)(((y0 + z_oy) * Wd + x0 + z_ox) * ELEM) : kOOB;
 
-    constexpr int LEAD = ADJ ? 2 * HH : HH;
-    const int zlo = max(z0 - LEAD, 0);
-    const int zhi = ADJ ? z1 + 3 + 2 * HH : z1 + 1 + HH;
-    const int zc_lo = ADJ ? max(z0 - HH, 0) : z0;
-    const int zc_hi = ADJ ? min(z1 + HH, D) : z1;
+    const int zlo = max(z0 - 2 * HH, 0);
+    const int zhi = z1 + 3 + 2 * HH;
+    const int zc_lo = max(z0 - HH, 0);
+    const int zc_hi = min(z1 + HH, D);
 
     // F state: the ring of the last k planes' p,t (slot r = position of the plane in its block of
     // k), the prefix sums of the five fields over the current block, and p,t of the next plane
@@ -341,7 +276,6 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
         float adj[NADJ][G::SY];  // alpha, beta, gamma (and alpha', beta') of the segment's outputs
 #pragma unroll
         for (int i = 0; i < G::SY; ++i) {
-            const int ay = y_start + i;
             const float Sp = S[0][i], St = S[1][i], Spp = S[2][i], Stt = S[3][i], Spt = S[4][i];
             const float X = fmaf(-Sp, St, nf * Spt);
             // n dr is added after the cancellation: folded into the fma that rounds n Spp, it
@@ -355,41 +289,25 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
             const bool live = y_inv[i] && (ncc < 1.0f);
             const float nccc = (ncc >= 1.0f) ? 1.0f : ncc;
             if (y_core[i]) lsum += nccc;
-            if constexpr (ADJ) {
-                // masking cr masks all three coefficients (alpha, beta, gamma are multiples of it)
-                const float crm = live ? cr : 0.f;
-                const float uu = crm * VT;
-                const float w = fmaf(-Sp, uu, St);
-                adj[0][i] = crm * w;
-                adj[1][i] = crm * uu;
-                adj[2][i] = crm;
-                if constexpr (DUAL) {
-                    // the target's: u' = (c/s)(VP s), w' = Sp - St u' (the swapped pass's uu, w)
-                    const float uu2 = crm * (VP * VS);
-                    adj[3][i] = crm * fmaf(-St, uu2, Sp);
-                    adj[4][i] = crm * uu2;
-                }
-                if constexpr (!G::ASWAP) {
-#pragma unroll
-                    for (int c = 0; c < NADJ; ++c) Gs[y_go + c * G::GP + i * G::GST] = adj[c][i];
-                }
+            // masking cr masks all three coefficients (alpha, beta, gamma are multiples of it)
+            const float crm = live ? cr : 0.f;
+            const float uu = crm * VT;
+            const float w = fmaf(-Sp, uu, St);
+            adj[0][i] = crm * w;
+            adj[1][i] = crm * uu;
+            adj[2][i] = crm;
+            if constexpr (DUAL) {
+                // the target's: u' = (c/s)(VP s), w' = Sp - St u' (the swapped pass's uu, w)
+                const float uu2 = crm * (VP * VS);
+                adj[3][i] = crm * fmaf(-St, uu2, Sp);
+                adj[4][i] = crm * uu2;
             }
-            if constexpr (MODE == MODE_MAPS) {
-                if (count && y_core[i]) {
-                    const float uu = cr * VT;
-                    const float w = fmaf(-Sp, uu, St);
-                    const int gx = x0 - HH + y_ax, gy = y0 - HH + ay;
-                    const int64_t o = ((b * D + zcY) * Hd + gy) * (int64_t)Wd + gx;
-                    a.ncc_map[o] = nccc;
-                    if (a.a_map) {  // null: the ncc map alone
-                        a.a_map[o] = live ? (-2.f * VS) * (cr * w) : 0.f;
-                        a.b_map[o] = live ? (-nf * VS) * (cr * uu) : 0.f;
-                        a.c_map[o] = live ? (2.f * nf * VS) * cr : 0.f;
-                    }
-                }
+            if constexpr (!G::ASWAP) {
+#pragma unroll
+                for (int c = 0; c < NADJ; ++c) Gs[y_go + c * G::GP + i * G::GST] = adj[c][i];
             }
         }
-        if constexpr (ADJ && G::ASWAP) {  // Gs rows along y: one float4 per field
+        if constexpr (G::ASWAP) {  // Gs rows along y: one float4 per field
             static_assert(G::SY == 4, "float4 rows");
 #pragma unroll
             for (int c = 0; c < NADJ; ++c)
@@ -403,12 +321,11 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
     // (inactive ones through a zero-sized buffer), so the number of outstanding memory operations
     // is the same on every path and the waits before use stay exact. With STORE the z-sums go to
     // the LDS column by column as they are formed; without, f_store writes them later.
-    // F's columns [JB, JE) of this lane (f_sums runs them all, then the prefetch)
-    auto f_cols = [&](auto rc, auto store, auto jb, auto je) __attribute__((always_inline)) {
+    auto f_cols = [&](auto rc, auto store) __attribute__((always_inline)) {
         constexpr int r = decltype(rc)::value;
         constexpr bool STORE = decltype(store)::value;
 #pragma unroll
-        for (int j = decltype(jb)::value; j < decltype(je)::value; ++j) {
+        for (int j = 0; j < J; ++j) {
             if (j > 0 && !f_col1) continue;
             zstep5<K, r, F_CHAIN>(pnext[j], tnext[j], fpre[j], pring[j], tring[j], fch[j], zsum[j]);
             if constexpr (STORE) {
@@ -430,7 +347,7 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
         fta += PB;
     };
     auto f_sums = [&](auto rc, auto store, int zi) __attribute__((always_inline)) {
-        f_cols(rc, store, std::integral_constant<int, 0>{}, std::integral_constant<int, J>{});
+        f_cols(rc, store);
         f_pref(zi);
     };
     auto f_store = [&]() __attribute__((always_inline)) {
@@ -466,14 +383,8 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
     // advanced in place leave about 55; with the row waits moved behind F, (2,16,128^3) went from
     // 0.344 / 0.369 / 0.401 / 0.584 to 0.331 / 0.359 / 0.391 / 0.564 ms at k = 3 / 5 / 7 / 9.
     constexpr int Y_EARLY = DUAL ? (HH <= 1 ? 5 : HH == 2 ? (BF16 ? 2 : 0) : 0)
-                                 : !ADJ ? (HH <= 2 ? 5 : HH == 3 ? 3 : 0)
                                  : HH <= 1 ? 5 : HH == 2 ? 3 : HH == 3 ? 2 : 0;   // Y rows read before F
     constexpr bool F_STORE_AT_ONCE = Y_EARLY < 5;
-    // Y_MID of Y's rows are read between F's two columns, after the box sums of the early rows
-    // (whose registers they take); the rest after F. k = 9 without the adjoint: one row; with it, none
-    // (the row spills registers, 3% slower).
-    constexpr int Y_MID = HH == 4 && J == 2 && !ADJ ? 1 : 0;
-    static_assert(Y_EARLY + Y_MID <= 5, "Y rows");
     constexpr bool AX_EARLY = HH <= 2 && !DUAL;               // the AX row read before F
     constexpr int NY = G::SY + 2 * HH, NA = G::SA + 2 * HH, NX = G::SX + 2 * HH, NB = G::SB + 2 * HH;
     // P0's early reads (Y's first rows or the AX row) share one register array: the two kinds of
@@ -488,7 +399,7 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
             const int zcY = zi - 1 - HH;   // the plane Y(zi-1) is centred on (the z-sums of F(z): z-h)
             const uint32_t t = (uint32_t)(zi - tb);
             const bool do_x = t < n_x, do_y = t - 1u < n_y, do_a = t - 2u < n_a, do_b = t - 2u < n_b;
-            const bool actA = ADJ && t - 3u < nz;   // the xy-sums AZ(zi-3) reads
+            const bool actA = t - 3u < nz;   // the xy-sums AZ(zi-3) reads
 
             // ============================ phase P0 ============================
             // AZ(zi-3) reads, Y(zi-1) y-sums, AX(zi-2), F(zi), AZ(zi-3)
@@ -503,7 +414,7 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
                     ys[c] = actA ? gy : 0.f;
                 }
             };
-            if constexpr (ADJ && HH <= 3) az_read();
+            if constexpr (HH <= 3) az_read();
             lds_f4 eq[NEQ];
             lds_f2 eh[NEH];
             if (do_y) {
@@ -513,37 +424,14 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
                 row_load<NA>(Gs + a_src, eq, eh[0]);
             }
             float S[5][G::SY];  // Y's box sums, carried into P1
-            lds_f4 mq[cmax(Y_MID * YQ, 1)];
-            lds_f2 mh[cmax(Y_MID, 1)];
-            if constexpr (Y_MID > 0) {
-                // F's first column; then the box sums of the early rows and the reads of the mid
-                // rows; then F's second column and the prefetch
-                f_cols(rc, std::true_type{}, std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{});
-                if (do_y) {
-#pragma unroll
-                    for (int q = 0; q < Y_EARLY; ++q) {
-                        float v[NY];
-                        row_take<NY>(eq + q * YQ, eh[q], v);
-                        box_sums<HH, G::SY>(v, S[q]);
-                    }
-#pragma unroll
-                    for (int q = 0; q < Y_MID; ++q)
-                        row_load<NY>(Xs + (Y_EARLY + q) * G::XP + y_xo, mq + q * YQ, mh[q]);
-                }
-                f_cols(rc, std::true_type{}, std::integral_constant<int, 1>{}, std::integral_constant<int, J>{});
-                f_pref(zi);
-            } else {
-                f_sums(rc, std::integral_constant<bool, F_STORE_AT_ONCE>{}, zi);
-            }
+            f_sums(rc, std::integral_constant<bool, F_STORE_AT_ONCE>{}, zi);
             if (do_y) {
-                // the rows not yet summed: early rows (held in er), mid rows (em), the rest read now
+                // the early rows (held in eq, eh), the rest read now
 #pragma unroll
-                for (int q = Y_MID > 0 ? Y_EARLY : 0; q < 5; ++q) {
+                for (int q = 0; q < 5; ++q) {
                     float v[NY];
                     if (q < Y_EARLY) {
                         row_take<NY>(eq + q * YQ, eh[q < Y_EARLY ? q : 0], v);
-                    } else if (q < Y_EARLY + Y_MID) {
-                        row_take<NY>(mq + (q - Y_EARLY) * YQ, mh[q < Y_EARLY + Y_MID ? q - Y_EARLY : 0], v);
                     } else {
                         lds_row(Xs + q * G::XP + y_xo, v);
                     }
@@ -562,8 +450,8 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
                 for (int i = 0; i < G::SA; ++i) GXs[a_dst + i * G::GXS] = o[i];
             }
             if constexpr (!F_STORE_AT_ONCE) f_store();
-            if constexpr (ADJ && HH > 3) az_read();
-            if constexpr (ADJ) {
+            if constexpr (HH > 3) az_read();
+            {
                 // AZ(zi-3): z-sums of the xy-sums over the k planes of the output plane zo = the
                 // prefix of the current block plus the previous block's suffix (ring and chain)
                 // (lanes without an output column run on a clamped one and store out of range,
@@ -630,7 +518,6 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
     }
 
     // ---- workgroup partial of the ncc sum: wave64 reduction, then the waves in fixed order
-    if constexpr (MODE == MODE_MAPS) return;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) loss_acc += __shfl_xor(loss_acc, off, 64);
     const int lane = HH >= 3 ? (int)__lane_id() : (tid & 63);
@@ -649,12 +536,8 @@ template <int HH>
 hipError_t launch_fused(int mode, bool bf16, const FusedArgs& a, uint32_t nblocks, hipStream_t st) {
     const dim3 grid(nblocks), block(NT);
 #define FL_LAUNCH(BF, MD) hipLaunchKernelGGL((lncc_fused_kernel<HH, BF, MD>), grid, block, 0, st, a)
-    if (mode == MODE_LOSS) {
-        if (bf16) FL_LAUNCH(true, MODE_LOSS); else FL_LAUNCH(false, MODE_LOSS);
-    } else if (mode == MODE_GRAD) {
+    if (mode == MODE_GRAD) {
         if (bf16) FL_LAUNCH(true, MODE_GRAD); else FL_LAUNCH(false, MODE_GRAD);
-    } else if (mode == MODE_MAPS) {
-        if (bf16) FL_LAUNCH(true, MODE_MAPS); else FL_LAUNCH(false, MODE_MAPS);
     } else if (mode == MODE_DUAL) {
         if (bf16) FL_LAUNCH(true, MODE_DUAL); else FL_LAUNCH(false, MODE_DUAL);
     } else {

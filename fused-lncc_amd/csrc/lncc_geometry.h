@@ -132,6 +132,29 @@ struct Geo {
     static_assert(LDS_FLOATS * 4 <= 160 * 1024, "LDS");
 };
 
+// ---- the forward-only kernel (lncc_forward_kernel.h): NC columns per F lane, 16 lanes per row.
+template <int H, int NC>
+struct FwdGeo {
+    static constexpr int SY = 4;                                    // output rows per Y lane
+    static constexpr int RW = 16 * NC, ADV = RW - 2 * H;            // tile width, distance of tiles
+    static constexpr int YSEG = NC == 3 ? 8 : 7, OY = YSEG * SY;    // output rows of a tile
+    static constexpr int IY = OY + 2 * H, NFW = cdiv(IY, 4), NYW = cdiv(RW * YSEG, 64);
+    static constexpr int LANES = 64 * (NFW + NYW);
+    // Xs[buffer][plane][field][j * 16 + l][iy]: rows along y, row j * 16 + l is column NC l + j. A row
+    // stride of 2 mod 4 floats spreads a half-wave's stores (16 lanes of one column each, two rows iy)
+    // over the 32 banks, and the Y lanes' 64-bit reads from row to row; a stride of 4 mod 8, which
+    // 128-bit reads would need, makes the stores conflict 2-way. Fields a multiple of 64 floats apart
+    // pair into write2st64 where that fits.
+    static constexpr int XS = IY + (6 - IY % 4) % 4, XP0 = RW * XS;
+    static constexpr bool fits(int planes, int xp) { return (2 * planes * 5 * xp + 2 * NYW) * 4 <= 160 * 1024; }
+    // planes per barrier: two at k = 9 (10% faster there; below, no gain for long marches and a longer
+    // lead-in for short ones)
+    static constexpr int PPB = H == 4 ? 2 : 1;
+    static constexpr int XP = fits(PPB, rup64(XP0)) ? rup64(XP0) : XP0;
+    static constexpr int PLANE = 5 * XP, BUF = PPB * PLANE;
+    static_assert(NYW * 64 == RW * YSEG && LANES <= 1024 && XS % 4 == 2 && fits(PPB, XP), "lanes");
+};
+
 // ---- the small-volume kernel (lncc_small.hip): one workgroup of kSmallLanes lanes per volume
 // whose D, H, W are all at most kSmallEdge, the volume zero-padded to kSmallEdge^3 in LDS. Lanes
 // form four quarters q (whole waves) of 16 x 16; a quarter owns positions 4q..4q+3 of a line and

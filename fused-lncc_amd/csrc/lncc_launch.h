@@ -7,8 +7,9 @@
 
 namespace fl {
 
-// LOSS: partial sums only; GRAD: and the pred gradient; MAPS: the reference's four maps; DUAL:
-// the partial sums and both gradients (the marching kernel only)
+// LOSS: partial sums only and MAPS: the reference's four maps (forward-only and small-volume
+// kernels); GRAD: the partial sums and the pred gradient (fused and small-volume kernels); DUAL: and
+// both gradients (fused kernel)
 enum Mode { MODE_LOSS = 0, MODE_GRAD = 1, MODE_MAPS = 2, MODE_DUAL = 3 };
 
 struct FusedArgs {
@@ -23,6 +24,8 @@ struct FusedArgs {
     double* partials; // one ncc partial sum per workgroup
     int dimD, dimH, dimW;
     int ntx, nty, nzc, dchunk;
+    uint32_t nparts;          // forward-only kernel: the partials that the reduction reads (>= the grid),
+    uint32_t npieces;         // and its pieces (lncc_forward_kernel.h)
     float inv_n, nf, ndr;     // 1/n, n = k^3 and n * smooth_dr as float32
     float gscale;             // (2 n / M) s, s = range_scale(k) (the kernel's adjoints carry 1/s)
 };
@@ -43,6 +46,10 @@ hipError_t launch_fused_h1(int mode, bool bf16, const FusedArgs& a, uint32_t nbl
 hipError_t launch_fused_h2(int mode, bool bf16, const FusedArgs& a, uint32_t nblocks, hipStream_t st);
 hipError_t launch_fused_h3(int mode, bool bf16, const FusedArgs& a, uint32_t nblocks, hipStream_t st);
 hipError_t launch_fused_h4(int mode, bool bf16, const FusedArgs& a, uint32_t nblocks, hipStream_t st);
+
+// The forward-only kernel (lncc_forward.hip), MODE_LOSS and MODE_MAPS: `cols` input columns per F lane
+// (forward_width lists the widths of a halo).
+hipError_t launch_forward(int halo, int cols, int mode, bool bf16, const FusedArgs& a, uint32_t nblocks, hipStream_t st);
 
 // The small-volume kernel (lncc_small.hip): volumes whose D, H and W are all at most kSmallEdge
 // (lncc_geometry.h), one workgroup of kSmallLanes lanes per volume (FusedArgs' tile and chunk
