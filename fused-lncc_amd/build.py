@@ -1,7 +1,8 @@
-"""Build libfused_lncc_hip.so for gfx950 in-tree: one hipcc job per translation unit, then link.
+"""Build libfused_lncc_hip.so for gfx950 in-tree: one hipcc job per translation unit, then link; and
+_step.so, the eager step as a torch extension (host code only), with the host compiler.
 
-Usage: ``python fused-lncc_amd/build.py [--jobs N]``. The library lands next to the Python package
-(``fused-lncc_amd/fused_lncc/libfused_lncc_hip.so``), objects under ``fused-lncc_amd/_build/``.
+Usage: ``python fused-lncc_amd/build.py [--jobs N]``. Both land next to the Python package
+(``fused-lncc_amd/fused_lncc/``), objects under ``fused-lncc_amd/_build/``.
 """
 import argparse
 import concurrent.futures as cf
@@ -33,11 +34,32 @@ def _compile(src):
     return obj
 
 
+def _build_step():
+    """_step.so (csrc/torch_step.cpp) against the installed torch's headers and libraries. The torch
+    libraries are found where torch loaded them from when the module is imported."""
+    import sysconfig
+    import torch
+    root = os.path.dirname(torch.__file__)
+    inc = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+           os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"), sysconfig.get_paths()["include"]]
+    out = os.path.join(os.path.dirname(LIB), "_step.so")
+    cmd = ([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__"]
+           + [a for i in inc for a in ("-isystem", i)] + [os.path.join(CSRC, "torch_step.cpp"), "-o", out + ".tmp"]
+           + ["-L" + os.path.join(root, "lib"), "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", "-lc10_hip"])
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("building _step.so failed:\n" + r.stdout + r.stderr)
+    os.replace(out + ".tmp", out)
+
+
 def build(jobs=None, verbose=True):
     os.makedirs(BUILD, exist_ok=True)
-    jobs = jobs or min(len(SOURCES), os.cpu_count() or 1)
+    jobs = jobs or min(len(SOURCES) + 1, os.cpu_count() or 1)
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
+        step = ex.submit(_build_step)
         objs = list(ex.map(_compile, SOURCES))
+        step.result()
     tmp = LIB + ".tmp"
     cmd = [HIPCC, "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", tmp] + objs
     r = subprocess.run(cmd, capture_output=True, text=True)

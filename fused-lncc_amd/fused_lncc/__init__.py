@@ -99,6 +99,18 @@ def _traced(t):
     return type(t) is not torch.Tensor and torch._guards.detect_fake_mode((t,)) is not None
 
 
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def _watched():
+    """True where something observes or transforms the call: a trace or compilation, a dispatch or
+    function mode, a functorch transform, forward-mode differentiation. The Python autograd function
+    then runs, which all of them know how to treat (or to refuse)."""
+    return (_compiling() or torch._C._len_torch_dispatch_stack() > 0 or torch._C._len_torch_function_stack() > 0
+            or torch._C._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0
+            or torch._C._get_tracing_state() is not None)
+
+
 class _FusedLNCC(torch.autograd.Function):
     """Autograd wrapper: the gradient is produced in forward by the fused kernel and handed out in
     backward (fused_lncc/__init__.py:49-74 computes it in backward from four saved fp32 maps).
@@ -210,6 +222,12 @@ def fused_lncc_loss(pred, target, kernel_size=7, smooth_dr=1e-5, *, target_grad=
     (2,16,128^3) k=7); volumes of at most 16^3 take a second pass with pred and target swapped."""
     assert pred.dim() == 5 and pred.shape == target.shape, "expect matching (N,C,D,H,W)"
     assert kernel_size % 2 == 1, "kernel_size must be odd"
+    if type(pred) in _PLAIN and type(target) in _PLAIN and not _watched():
+        step = _lib.eager_step()
+        if step is not None:
+            loss = step(pred, target, int(kernel_size), float(smooth_dr), bool(target_grad))
+            if loss is not None:
+                return loss
     # The gradient is computed in the forward kernel only when autograd will ask for it; under
     # no_grad or for a pred without requires_grad the kernel reads 8 B/voxel and writes nothing.
     grad_on = torch.is_grad_enabled()

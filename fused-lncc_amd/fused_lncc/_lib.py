@@ -103,6 +103,29 @@ def load():
     return _lib
 
 
+# The C ABI functions that the eager step (csrc/torch_step.cpp) calls, in the order of its init().
+_STEP_API = ("fl_validate", "fl_workspace_bytes", "fl_lncc_loss_grad", "fl_lncc_loss_grad_pt", "fl_scale_grad",
+             "fl_last_error")
+_step = None   # the extension's step(), False where it cannot be loaded
+
+
+def eager_step():
+    """step() of the eager-step extension, bound to the loaded library, or None where the extension is
+    not there (or was built for another torch): the Python autograd function then does the same."""
+    global _step
+    if _step is None:
+        lib = load()
+        try:
+            from . import _step as ext_module
+            ext_module.init(*[ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in _STEP_API])
+            _step = ext_module.step
+        except ImportError as e:
+            print(f"fused_lncc: the eager-step extension is not used ({e}); run `python fused-lncc_amd/build.py`",
+                  file=sys.stderr, flush=True)
+            _step = False
+    return _step or None
+
+
 class dchunk:
     """Test hook: launches on this thread inside the block split D into chunks of `planes` output
     planes (clamped to D); the launch planner decides again on exit."""

@@ -1,0 +1,175 @@
+"""The eager step extension against the Python autograd function, call by call: the same bits, the same
+gradients handed out, the same refusals; and the calls that are to keep the Python function."""
+import contextlib
+
+import pytest
+import torch
+
+import fused_lncc
+import workloads as wl
+from fused_lncc import _lib, fused_lncc_loss
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@contextlib.contextmanager
+def python_path(monkeypatch):
+    with monkeypatch.context() as m:
+        m.setattr(_lib, "_step", False)
+        yield
+
+
+def both(monkeypatch, f):
+    """f() through the extension and through the Python function."""
+    assert _lib.eager_step() is not None
+    got = f()
+    with python_path(monkeypatch):
+        want = f()
+    return got, want
+
+
+def pair(shape=(2, 2, 9, 20, 24), dtype=torch.float32, seed=3):
+    p, t = wl.randn_pair(shape, seed)
+    return p.to(dtype).to(DEV), t.to(dtype).to(DEV)
+
+
+def same(a, b):
+    assert (a is None) == (b is None)
+    if a is not None:
+        assert a.dtype == b.dtype and a.shape == b.shape and a.requires_grad == b.requires_grad and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("k", [3, 9])
+@pytest.mark.parametrize("weight", [1.0, 0.25])
+@pytest.mark.parametrize("target_grad", [False, True])
+@pytest.mark.parametrize("shape", [(2, 2, 9, 20, 24), (3, 1, 8, 7, 6)])
+def test_step(monkeypatch, dtype, k, weight, target_grad, shape):
+    def f():
+        p, t = pair(shape, dtype)
+        p.requires_grad_(True)
+        t.requires_grad_(True)
+        loss = fused_lncc_loss(p, t, k, 1e-4, target_grad=target_grad)
+        (weight * loss).backward()
+        return loss.detach(), p.grad, t.grad
+    for a, b in zip(*both(monkeypatch, f)):
+        same(a, b)
+
+
+@pytest.mark.parametrize("pg,tg,on", [(False, False, True), (False, True, True), (True, False, False), (True, True, True)])
+@pytest.mark.parametrize("target_grad", [False, True])
+def test_what_requires_grad(monkeypatch, pg, tg, on, target_grad):
+    def f():
+        p, t = pair()
+        p.requires_grad_(pg)
+        t.requires_grad_(tg)
+        with torch.set_grad_enabled(on):
+            loss = fused_lncc_loss(p, t, 5, target_grad=target_grad)
+        if loss.requires_grad:
+            loss.backward()
+        return loss, p.grad, t.grad
+    for a, b in zip(*both(monkeypatch, f)):
+        same(a, b)
+
+
+def test_views_and_non_leaves(monkeypatch):
+    def f():
+        p, t = pair((1, 4, 10, 12, 14))
+        x = p.requires_grad_(True)
+        loss = fused_lncc_loss((2 * x).transpose(3, 4), t.transpose(3, 4), 7)   # contiguous copies, through autograd
+        loss.backward()
+        q = p.detach()[:, 1:3].requires_grad_(True)                             # a view at an offset
+        fused_lncc_loss(q, t[:, 1:3], 7).backward()
+        return loss.detach(), x.grad, q.grad
+    for a, b in zip(*both(monkeypatch, f)):
+        same(a, b)
+
+
+@pytest.mark.parametrize("target_grad", [False, True])
+def test_retained_graph_recomputes(monkeypatch, target_grad):
+    def f():
+        p, t = pair()
+        p.requires_grad_(True)
+        t.requires_grad_(target_grad)
+        loss = fused_lncc_loss(p, t, 7, target_grad=target_grad)
+        wrt = (p, t) if target_grad else (p,)
+        first = torch.autograd.grad(loss, wrt, retain_graph=True)
+        second = torch.autograd.grad(3.0 * loss, wrt)
+        with pytest.raises(RuntimeError, match="second time"):
+            torch.autograd.grad(loss, wrt)
+        return first + second
+    for a, b in zip(*both(monkeypatch, f)):
+        same(a, b)
+
+
+def test_inputs_changed_in_place(monkeypatch):
+    """The first backward hands out what the forward formed; one that recomputes refuses inputs that
+    were changed since."""
+    def f():
+        p, t = pair()
+        x = p.requires_grad_(True) * 1.0
+        loss = fused_lncc_loss(x, t, 7)
+        t.add_(1.0)
+        (g,) = torch.autograd.grad(loss, x, retain_graph=True)
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            torch.autograd.grad(loss, x)
+        return (g,)
+    for a, b in zip(*both(monkeypatch, f)):
+        same(a, b)
+
+
+def test_hooks_create_graph_and_streams(monkeypatch):
+    def f():
+        seen = []
+        p, t = pair()
+        p.requires_grad_(True)
+        with torch.autograd.graph.saved_tensors_hooks(lambda x: (seen.append(x.shape), x.clone())[1], lambda x: x):
+            loss = fused_lncc_loss(p, t, 7)
+        torch.autograd.grad(loss, p, retain_graph=True)
+        (again,) = torch.autograd.grad(loss, p, create_graph=True)
+        s = torch.cuda.Stream()
+        s.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(s):
+            side = fused_lncc_loss(p, t, 7)
+            side.backward()
+        torch.cuda.current_stream().wait_stream(s)
+        return (torch.tensor(len(seen)), again.detach(), torch.tensor(again.requires_grad), side.detach(), p.grad)
+    for a, b in zip(*both(monkeypatch, f)):
+        same(a, b)
+
+
+def test_refusals_are_the_python_functions(monkeypatch):
+    p, t = pair()
+    for bad in (lambda: fused_lncc_loss(p.double(), t.double(), 7), lambda: fused_lncc_loss(p, t.bfloat16(), 7),
+                lambda: fused_lncc_loss(p.cpu(), t.cpu(), 7), lambda: fused_lncc_loss(p, t, 11),
+                lambda: fused_lncc_loss(p, t.cpu(), 7), lambda: fused_lncc_loss(p[:, :0], t[:, :0], 7)):
+        def f():
+            with pytest.raises(RuntimeError) as e:
+                bad()
+            return type(e.value), str(e.value)
+        got, want = both(monkeypatch, f)
+        assert got == want
+
+
+def test_watched_calls_keep_the_python_function(monkeypatch):
+    calls = []
+    step = _lib.eager_step()
+    monkeypatch.setattr(_lib, "_step", lambda *a: (calls.append(1), step(*a))[1])
+    p, t = pair()
+    fused_lncc_loss(p, t, 7)
+    assert len(calls) == 1
+
+    class Mode(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    with Mode():
+        fused_lncc_loss(p, t, 7)
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(lambda a, b: fused_lncc_loss(a, b, 7))(p[None], t[None])
+    with torch.autograd.forward_ad.dual_level():
+        d = torch.autograd.forward_ad.make_dual(p, torch.ones_like(p))
+        with pytest.raises((RuntimeError, NotImplementedError)):
+            fused_lncc_loss(d, t, 7)
+    assert fused_lncc._watched() is False and len(calls) == 1
