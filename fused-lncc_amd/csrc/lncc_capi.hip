@@ -50,7 +50,7 @@ int device_cus() {
 }
 
 // Workgroups: B volumes x (W/TX) x (H/TY) tiles x D-chunks. A chunk of d output planes costs
-// d + 4h + 3 pipeline steps (it recomputes the halo planes of its neighbours), so D is split only
+// d + 2h + 4 pipeline steps (it recomputes the halo planes of its neighbours), so D is split only
 // where that shortens the launch: small volumes, whose tiles alone leave CUs idle, get short chunks.
 // fl_test_set_dchunk fixes the chunk length for the calling thread (tests of chunk seams and of
 // long unsplit marches).
@@ -71,7 +71,7 @@ Plan plan_fused(int64_t B, int64_t D, int64_t H, int64_t W, int halo) {
     // callers pass shapes that passed check_grid, so base < 2^32 / NT; a forced chunk length can
     // multiply it by up to D <= 2^30, which still fits int64
     const int64_t base = B * p.ntx * p.nty;
-    // Split D into nzc chunks. A chunk of d planes costs d + 4h + 3 pipeline steps, and the
+    // Split D into nzc chunks. A chunk of d planes costs d + 2h + 4 pipeline steps, and the
     // workgroups run in rounds of one per CU: pick the split with the fewest rounds x steps (ties:
     // fewer workgroups).
     const int64_t kCUs = device_cus();
@@ -79,7 +79,7 @@ Plan plan_fused(int64_t B, int64_t D, int64_t H, int64_t W, int halo) {
     for (int64_t nzc = 1; nzc <= D; ++nzc) {
         const int64_t d = (D + nzc - 1) / nzc;
         const int64_t blocks = base * ((D + d - 1) / d);
-        const int64_t cost = ((blocks + kCUs - 1) / kCUs) * (d + 4 * halo + 3);
+        const int64_t cost = ((blocks + kCUs - 1) / kCUs) * (d + 2 * halo + 4);
         if (best_cost < 0 || cost < best_cost) {
             best_cost = cost;
             dchunk = d;
@@ -100,8 +100,8 @@ struct ForwardPlan {
     int64_t npieces, nblocks;
 };
 
-// The best split of tiles of one width, if better than `best`: a chunk of d planes costs d + 2h + 1
-// planes of cost `step`, and the workgroups, one per CU, take the chunks in rounds. Never more
+// The best split of tiles of one width, if better than `best`: a chunk of d planes costs d + 3
+// planes of cost `step` (the last step and the first loads), and the workgroups, one per CU, take the chunks in rounds. Never more
 // workgroups than the gradient plan's `gblocks`, whose count the reduction of the partial sums reads.
 template <int H, int NC>
 void try_forward(int64_t B, int64_t D, int64_t H_, int64_t W, int64_t gblocks, double step, ForwardPlan& f, double& best) {
@@ -111,7 +111,7 @@ void try_forward(int64_t B, int64_t D, int64_t H_, int64_t W, int64_t gblocks, d
     for (int64_t nzc = 1; nzc <= D; ++nzc) {
         const int64_t d = t_dchunk_override > 0 ? std::min(t_dchunk_override, D) : (D + nzc - 1) / nzc;
         const int64_t n = (D + d - 1) / d, pieces = tiles * n;
-        const double cost = (double)((pieces + most - 1) / most) * (double)(d + 2 * H + 1) * step;
+        const double cost = (double)((pieces + most - 1) / most) * (double)(d + 3) * step;
         if (best < 0 || cost < best) {
             best = cost;
             f = ForwardPlan{NC, (int)ntx, (int)nty, (int)n, (int)d, pieces, std::min(pieces, most)};

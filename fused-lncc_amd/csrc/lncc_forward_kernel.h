@@ -157,8 +157,8 @@ __global__ __launch_bounds__((FwdGeo<HH, NC>::LANES), 1) void lncc_forward_kerne
         int64_t b;
         int x0, y0;
         tile_origin<G>(a, tile, b, x0, y0);
-        // F runs planes [zlo, zend), Y one step (PPB planes) later
-        const int zlo = max(z0 - HH, 0), zend = z1 + HH, nsteps = (zend - zlo + G::PPB - 1) / G::PPB + 1;
+        // F runs planes [tb, zend), whose windows are centred on [z0, z1), Y one step (PPB planes) later
+        const int tb = z0 + HH, zend = z1 + HH, nsteps = (z1 - z0 + G::PPB - 1) / G::PPB + 1;
         const int gy = y0 - HH + iy, gx = x0 + NC * l;
         const bool row_in = gy >= 0 && gy < Hd;
         const uint32_t plane_bytes = (uint32_t)(HW * ELEM);
@@ -174,11 +174,12 @@ __global__ __launch_bounds__((FwdGeo<HH, NC>::LANES), 1) void lncc_forward_kerne
             for (int j = 1; j < NC; ++j) voff[j] = j < inside ? at + j * ELEM : kOOB;
         }
         const uint64_t PB = (uint64_t)HW * ELEM;
-        const uint64_t first = (uint64_t)(b * D + zlo) * PB;
+        // the ring's planes before the first: tb - K + 1 ... (possibly below 0: zero-sized)
+        const int64_t first = (b * D + tb - K + 1) * (int64_t)PB;
         uint64_t pa = (uint64_t)(uintptr_t)a.pred + first, ta = (uint64_t)(uintptr_t)a.target + first;
         float pn[2][NC], tn[2][NC];   // p, t of this plane and the next
         auto fetch = [&](int z, float (&p)[NC], float (&t)[NC]) __attribute__((always_inline)) {
-            const uint32_t n = z < min(D, zend) ? plane_bytes : 0u;
+            const uint32_t n = z >= 0 && z < min(D, zend) ? plane_bytes : 0u;
             const rsrc_words rp = words_at(pa, n), rt = words_at(ta, n);
             if (wide) {
                 load_run<NC>(rp, voff[0], p);
@@ -194,30 +195,47 @@ __global__ __launch_bounds__((FwdGeo<HH, NC>::LANES), 1) void lncc_forward_kerne
             pa += PB;
             ta += PB;
         };
-        fetch(zlo, pn[0], tn[0]);
-        fetch(zlo + 1, pn[1], tn[1]);
         float pring[NC][K], tring[NC][K], fpre[NC][5], ch[NC][5];
         constexpr int M = HH + 1;
         constexpr bool CH = HH >= 2 && NC * (2 * K + 10) <= 80;
+        // The march starts with a block: the k - 1 planes before its first one only enter windows, as
+        // the previous block, and go straight into their ring slots.
 #pragma unroll
-        for (int j = 0; j < NC; ++j)
+        for (int r = 1; r < K; ++r) {
+            float p[NC], t[NC];
+            fetch(tb - K + r, p, t);
 #pragma unroll
-            for (int s = 0; s < K; ++s) pring[j][s] = tring[j][s] = 0.f;
+            for (int j = 0; j < NC; ++j) {
+                pring[j][r] = p[j];
+                tring[j][r] = t[j];
+            }
+        }
+        fetch(tb, pn[0], tn[0]);
+        fetch(tb + 1, pn[1], tn[1]);
+        // the chain (zstep5): the previous block's sums over slots M .. K-1
+        auto form_chain = [&]() __attribute__((always_inline)) {
+            static_for<0, 5>([&](auto qc) __attribute__((always_inline)) {
+                constexpr int q = decltype(qc)::value;
 #pragma unroll
-        for (int j = 0; j < NC; ++j)
+                for (int j = 0; j < NC; ++j) {
+                    ch[j][q] = field<q>(pring[j][K - 1], tring[j][K - 1]);
 #pragma unroll
-            for (int q = 0; q < 5; ++q) ch[j][q] = 0.f;
+                    for (int s = K - 2; s >= M; --s) ch[j][q] = field_add<q>(ch[j][q], pring[j][s], tring[j][s]);
+                }
+            });
+        };
+        if constexpr (CH) form_chain();
         // The march is unrolled by 2 k: the ring slot is the plane's position in its block of k, the
         // buffers alternate with its parity.
         uint32_t buf = 0;   // LDS offset of the buffer being written
-        for (int base = zlo; base < zlo + nsteps * G::PPB; base += 2 * K) {
+        for (int base = tb; base < tb + nsteps * G::PPB; base += 2 * K) {
             static_for<0, 2 * K>([&](auto uc) __attribute__((always_inline)) {
                 constexpr int u = decltype(uc)::value, r = u % K, par = u % 2;
                 const int zi = base + u;
-                if (zi - u % G::PPB >= zlo + nsteps * G::PPB) return;   // whole steps
+                if (zi - u % G::PPB >= tb + nsteps * G::PPB) return;   // whole steps
                 float (&p)[NC] = pn[par];
                 float (&t)[NC] = tn[par];
-                const bool out = zi >= z0 + HH;   // before, the window's planes only enter the ring
+                const bool out = zi < zend;   // not in the last step, which is Y's alone
                 static_for<0, 5>([&](auto qc) __attribute__((always_inline)) {
                     constexpr int q = decltype(qc)::value;
                     float zs[NC];
@@ -245,17 +263,7 @@ __global__ __launch_bounds__((FwdGeo<HH, NC>::LANES), 1) void lncc_forward_kerne
                     pring[j][r] = p[j];
                     tring[j][r] = t[j];
                 }
-                if constexpr (CH && r == K - 1) {
-                    static_for<0, 5>([&](auto qc) __attribute__((always_inline)) {
-                        constexpr int q = decltype(qc)::value;
-#pragma unroll
-                        for (int j = 0; j < NC; ++j) {
-                            ch[j][q] = field<q>(pring[j][K - 1], tring[j][K - 1]);
-#pragma unroll
-                            for (int s = K - 2; s >= M; --s) ch[j][q] = field_add<q>(ch[j][q], pring[j][s], tring[j][s]);
-                        }
-                    });
-                }
+                if constexpr (CH && r == K - 1) form_chain();
                 fetch(zi + 2, p, t);
                 if constexpr (u % G::PPB == G::PPB - 1) {
                     __syncthreads();
@@ -280,7 +288,7 @@ __global__ __launch_bounds__((FwdGeo<HH, NC>::LANES), 1) void lncc_forward_kerne
         int64_t b;
         int x0, y0;
         tile_origin<G>(a, tile, b, x0, y0);
-        const int zlo = max(z0 - HH, 0), zend = z1 + HH, nsteps = (zend - zlo + G::PPB - 1) / G::PPB + 1;
+        const int nsteps = (z1 - z0 + G::PPB - 1) / G::PPB + 1;
         const int gx = x0 + x, gy = y0 + seg * G::SY;
         // a column is this tile's if both neighbours' columns of its window were there, or are outside
         // the volume
@@ -291,8 +299,8 @@ __global__ __launch_bounds__((FwdGeo<HH, NC>::LANES), 1) void lncc_forward_kerne
         uint32_t buf = G::BUF;   // the buffer written one step ago
         for (int st = 0; st < nsteps; ++st) {
             // the planes that this step's sums are centred on: zc .. zc + PPB - 1
-            const int zc = zlo + (st - 1) * G::PPB - HH;
-            if (zc + G::PPB > z0) {
+            const int zc = z0 + (st - 1) * G::PPB;
+            if (st > 0) {
                 const float* const row = xs + buf;
                 lds_f2 rows[G::PPB][5][NY / 2];
 #pragma unroll
@@ -308,7 +316,7 @@ __global__ __launch_bounds__((FwdGeo<HH, NC>::LANES), 1) void lncc_forward_kerne
                         pairs_take<NY>(rows[e][q], v);
                         box_sums<HH, G::SY>(v, S[q]);
                     }
-                    const bool count = zc + e >= z0 && zc + e < z1;
+                    const bool count = zc + e < z1;
                     float lsum = -0.f;
 #pragma unroll
                     for (int i = 0; i < G::SY; ++i) {

@@ -194,15 +194,17 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
     const bool z_in = has_z && x0 + z_ox < Wd && y0 + z_oy < Hd;
     const uint32_t z_voff = z_in ? (uint32_t)(((y0 + z_oy) * Wd + x0 + z_ox) * ELEM) : kOOB;
 
-    const int zlo = max(z0 - 2 * HH, 0);
     const int zhi = z1 + 3 + 2 * HH;
     const int zc_lo = max(z0 - HH, 0);
     const int zc_hi = min(z1 + HH, D);
+    const int tb = HH + zc_lo;   // the march's first plane: its z windows are the first that X needs
 
     // F state: the ring of the last k planes' p,t (slot r = position of the plane in its block of
     // k), the prefix sums of the five fields over the current block, and p,t of the next plane
-    // (prefetched one step ahead). The ring starts at zero: nothing before the first plane of the
-    // march enters a window that is used.
+    // (prefetched one step ahead). The march starts with a block: the k - 1 planes before its first
+    // one only enter windows, as the previous block, so they are loaded straight into their ring
+    // slots, all at once, and cost one memory latency instead of k - 1 steps of the pipeline (chunks
+    // of 4 planes at k = 7 took 19 steps, now 13: 96^3 25.2 -> 20.8 us with the drain steps' F left out).
     float pring[J][K], tring[J][K], fpre[J][5], fch[J][5], zsum[J][5], pnext[J], tnext[J];
     float pz = 0.f, tzz = 0.f;  // AZ: p,t at this step's output plane (prefetched one step ahead)
 #pragma unroll
@@ -213,19 +215,23 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
             fch[j][q] = 0.f;
             zsum[j][q] = 0.f;
         }
-#pragma unroll
-        for (int r = 0; r < K; ++r) {
-            pring[j][r] = 0.f;
-            tring[j][r] = 0.f;
-        }
+        pring[j][0] = 0.f;
+        tring[j][0] = 0.f;
     }
     {
-        const rsrc_words rp = words_at((uint64_t)(uintptr_t)pvol + (uint64_t)zlo * HW * ELEM, plane_bytes);
-        const rsrc_words rt = words_at((uint64_t)(uintptr_t)tvol + (uint64_t)zlo * HW * ELEM, plane_bytes);
+        const int64_t at = (int64_t)(tb - K + 1) * HW * ELEM;
+        uint64_t pa = (uint64_t)(uintptr_t)pvol + at, ta = (uint64_t)(uintptr_t)tvol + at;
 #pragma unroll
-        for (int j = 0; j < J; ++j) {
-            pnext[j] = load_elem<BF16>(rp, voff[j]);
-            tnext[j] = load_elem<BF16>(rt, voff[j]);
+        for (int r = 1; r <= K; ++r) {   // plane tb - K + r; r = K: the first plane of the march
+            const uint32_t n = (uint32_t)(tb - K + r) < (uint32_t)D ? plane_bytes : 0u;
+            const rsrc_words rp = words_at(pa, n), rt = words_at(ta, n);
+#pragma unroll
+            for (int j = 0; j < J; ++j) {
+                (r < K ? pring[j][r < K ? r : 0] : pnext[j]) = load_elem<BF16>(rp, voff[j]);
+                (r < K ? tring[j][r < K ? r : 0] : tnext[j]) = load_elem<BF16>(rt, voff[j]);
+            }
+            pa += (uint64_t)HW * ELEM;
+            ta += (uint64_t)HW * ELEM;
         }
     }
     // AZ state: the ring of the last k planes' xy-sums of the adjoint fields and their prefix sums
@@ -247,7 +253,7 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
     // range gets a zero-sized resource (its address is never dereferenced).
     constexpr int ZO = 3 + 2 * HH;
     const uint64_t PB = (uint64_t)HW * ELEM;
-    const int64_t fz = (int64_t)(zlo + 1) * (int64_t)PB, oz = (int64_t)(zlo - ZO) * (int64_t)PB;
+    const int64_t fz = (int64_t)(tb + 1) * (int64_t)PB, oz = (int64_t)(tb - ZO) * (int64_t)PB;
     uint64_t fpa = (uint64_t)(uintptr_t)pvol + fz, fta = (uint64_t)(uintptr_t)tvol + fz;
     uint64_t opa = (uint64_t)(uintptr_t)pvol + oz + PB, ota = (uint64_t)(uintptr_t)tvol + oz + PB;
     uint64_t oga = (uint64_t)(uintptr_t)gvol + oz, ogta = (uint64_t)(uintptr_t)gtvol + oz;
@@ -255,7 +261,6 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
     // Stage ranges: X(zi) runs for t = zi - HH - zc_lo in [0, nz), Y one step later, AX and AYs two,
     // AZ's input three: one subtraction and one unsigned compare each, zero planes for a wave
     // without the role.
-    const int tb = HH + zc_lo;
     const uint32_t nz = (uint32_t)(zc_hi - zc_lo);
     const uint32_t n_x = wave_x ? nz : 0u, n_y = wave_y ? nz : 0u, n_a = wave_a ? nz : 0u, n_b = wave_b ? nz : 0u;
     // z-window chains (zstep5 / zstep1): the previous block's sums over ring slots F_CHAIN..K-1
@@ -346,10 +351,6 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
         fpa += PB;
         fta += PB;
     };
-    auto f_sums = [&](auto rc, auto store, int zi) __attribute__((always_inline)) {
-        f_cols(rc, store);
-        f_pref(zi);
-    };
     auto f_store = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < J; ++j) {
@@ -385,6 +386,9 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
     constexpr int Y_EARLY = DUAL ? (HH <= 1 ? 5 : HH == 2 ? (BF16 ? 2 : 0) : 0)
                                  : HH <= 1 ? 5 : HH == 2 ? 3 : HH == 3 ? 2 : 0;   // Y rows read before F
     constexpr bool F_STORE_AT_ONCE = Y_EARLY < 5;
+    // no z-sums for the drain steps, which X does not read (2-5% at k >= 5; at k = 3 1% slower, and both
+    // gradients at k = 9, which spill, 8%)
+    constexpr bool F_STOP = HH >= 2 && !(DUAL && HH == 4);
     constexpr bool AX_EARLY = HH <= 2 && !DUAL;               // the AX row read before F
     constexpr int NY = G::SY + 2 * HH, NA = G::SA + 2 * HH, NX = G::SX + 2 * HH, NB = G::SB + 2 * HH;
     // P0's early reads (Y's first rows or the AX row) share one register array: the two kinds of
@@ -392,7 +396,7 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
     constexpr int YQ = row_quads(NY);
     constexpr int NEQ = cmax(cmax(Y_EARLY * YQ, AX_EARLY ? row_quads(NA) : 0), 1), NEH = cmax(Y_EARLY, 1);
 
-    for (int base = zlo; base < zhi; base += K) {
+    for (int base = tb; base < zhi; base += K) {
         static_for<0, K>([&](auto rc) __attribute__((always_inline)) {
             const int zi = base + decltype(rc)::value;
             if (zi >= zhi) return;
@@ -424,7 +428,8 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
                 row_load<NA>(Gs + a_src, eq, eh[0]);
             }
             float S[5][G::SY];  // Y's box sums, carried into P1
-            f_sums(rc, std::integral_constant<bool, F_STORE_AT_ONCE>{}, zi);
+            if (!F_STOP || t < nz) f_cols(rc, std::integral_constant<bool, F_STORE_AT_ONCE>{});
+            f_pref(zi);
             if (do_y) {
                 // the early rows (held in eq, eh), the rest read now
 #pragma unroll
