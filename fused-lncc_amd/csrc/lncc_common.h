@@ -61,6 +61,26 @@ __device__ __forceinline__ float load_elem(rsrc_words r, uint32_t voff) {
         return raw_load_f32(r, (int)voff, 0, AUX);
 }
 
+// The same load for a value that is used a step later: what the load leaves in its register (with
+// LATE, a bfloat16's bits), and the float it stands for. load_elem's conversion of a bfloat16 stands
+// where the load stands as far as the compiler is concerned, which then waits for the load at the end
+// of the step that issued it.
+template <bool LATE>
+using elem_raw = std::conditional_t<LATE, unsigned short, float>;
+template <bool BF16, bool LATE, int AUX = 0>
+__device__ __forceinline__ elem_raw<LATE> load_raw(rsrc_words r, uint32_t voff) {
+    static_assert(BF16 || !LATE, "float32 needs no conversion");
+    if constexpr (LATE)
+        return raw_load_b16(r, (int)voff, 0, AUX);
+    else
+        return load_elem<BF16, AUX>(r, voff);
+}
+__device__ __forceinline__ float widen(unsigned short bits) {
+    asm("" : "+v"(bits));   // here, not at the load
+    return __uint_as_float((uint32_t)bits << 16);
+}
+__device__ __forceinline__ float widen(float v) { return v; }
+
 // N = 3 or 4 consecutive floats in one load (4-byte aligned)
 template <int N>
 __device__ __forceinline__ void load_run(rsrc_words r, uint32_t voff, float (&v)[N]) {

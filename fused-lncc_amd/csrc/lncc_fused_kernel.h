@@ -205,8 +205,14 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
     // one only enter windows, as the previous block, so they are loaded straight into their ring
     // slots, all at once, and cost one memory latency instead of k - 1 steps of the pipeline (chunks
     // of 4 planes at k = 7 took 19 steps, now 13: 96^3 25.2 -> 20.8 us with the drain steps' F left out).
-    float pring[J][K], tring[J][K], fpre[J][5], fch[J][5], zsum[J][5], pnext[J], tnext[J];
-    float pz = 0.f, tzz = 0.f;  // AZ: p,t at this step's output plane (prefetched one step ahead)
+    // LATE: bfloat16 values prefetched for the next step are widened there, not before the barrier that
+    // ends this one, where the conversion waits for loads issued a phase ago. (2,16,128^3): k = 5 347 ->
+    // 337 us, both gradients at k = 9 981 -> 964 (160x192x224 127 -> 122); k = 9 within 0.5%. At k = 7,
+    // where it leaves the registers fuller, 1% slower, at k = 3 within 0.8% either way: as it was.
+    constexpr bool LATE = BF16 && (HH == 2 || HH == 4);
+    float pring[J][K], tring[J][K], fpre[J][5], fch[J][5], zsum[J][5];
+    elem_raw<LATE> pnext[J], tnext[J];
+    elem_raw<LATE> pz = 0, tzz = 0;  // AZ: p,t at this step's output plane (prefetched one step ahead)
 #pragma unroll
     for (int j = 0; j < J; ++j) {
 #pragma unroll
@@ -227,8 +233,13 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
             const rsrc_words rp = words_at(pa, n), rt = words_at(ta, n);
 #pragma unroll
             for (int j = 0; j < J; ++j) {
-                (r < K ? pring[j][r < K ? r : 0] : pnext[j]) = load_elem<BF16>(rp, voff[j]);
-                (r < K ? tring[j][r < K ? r : 0] : tnext[j]) = load_elem<BF16>(rt, voff[j]);
+                if (r < K) {
+                    pring[j][r < K ? r : 0] = load_elem<BF16>(rp, voff[j]);
+                    tring[j][r < K ? r : 0] = load_elem<BF16>(rt, voff[j]);
+                } else {
+                    pnext[j] = load_raw<BF16, LATE>(rp, voff[j]);
+                    tnext[j] = load_raw<BF16, LATE>(rt, voff[j]);
+                }
             }
             pa += (uint64_t)HW * ELEM;
             ta += (uint64_t)HW * ELEM;
@@ -332,7 +343,7 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
 #pragma unroll
         for (int j = 0; j < J; ++j) {
             if (j > 0 && !f_col1) continue;
-            zstep5<K, r, F_CHAIN>(pnext[j], tnext[j], fpre[j], pring[j], tring[j], fch[j], zsum[j]);
+            zstep5<K, r, F_CHAIN>(widen(pnext[j]), widen(tnext[j]), fpre[j], pring[j], tring[j], fch[j], zsum[j]);
             if constexpr (STORE) {
 #pragma unroll
                 for (int q = 0; q < 5; ++q) Zs[q * G::ZP + zaddr[j]] = zsum[j][q];
@@ -345,8 +356,8 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
         const rsrc_words rpn = words_at(fpa, nb), rtn = words_at(fta, nb);
 #pragma unroll
         for (int j = 0; j < J; ++j) {
-            pnext[j] = load_elem<BF16>(rpn, voff[j]);
-            tnext[j] = load_elem<BF16>(rtn, voff[j]);
+            pnext[j] = load_raw<BF16, LATE>(rpn, voff[j]);
+            tnext[j] = load_raw<BF16, LATE>(rtn, voff[j]);
         }
         fpa += PB;
         fta += PB;
@@ -466,7 +477,8 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
 #pragma unroll
                 for (int c = 0; c < NADJ; ++c) gw[c] = zstep1<K, r, A_CHAIN>(ys[c], gpre[c], gring[c]);
                 const int zo = zi - ZO;
-                const float g = a.gscale * fmaf(inv_n, gw[0], fmaf(pz, gw[1], -tzz * gw[2]));   // gscale holds s
+                const float po = widen(pz), to = widen(tzz);
+                const float g = a.gscale * fmaf(inv_n, gw[0], fmaf(po, gw[1], -to * gw[2]));   // gscale holds s
                 // Non-temporal: the gradient is never read back, and this re-read of p,t is the
                 // last use of those lines. With the default policy both would be promoted in the
                 // L2 and push out the planes that F loaded and this stage re-reads 2h+3 steps
@@ -479,15 +491,15 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
                 store_elem_buf<BF16, BF16 ? 0 : kNT>(words_at(oga, gb), z_voff, g);
                 oga += PB;
                 if constexpr (DUAL) {
-                    const float gt = a.gscale * fmaf(inv_n, gw[3], fmaf(tzz, gw[4], -pz * gw[2]));
+                    const float gt = a.gscale * fmaf(inv_n, gw[3], fmaf(to, gw[4], -po * gw[2]));
                     store_elem_buf<BF16, BF16 ? 0 : kNT>(words_at(ogta, gb), z_voff, gt);
                     ogta += PB;
                 }
                 // prefetch p,t at the next step's output plane; issued after this step's use, so
                 // one register each suffices and no copy has to wait for the load
                 const uint32_t ob = (uint32_t)(zo + 1 - z0) < (uint32_t)(z1 - z0) ? plane_bytes : 0u;
-                pz = load_elem<BF16, kNT>(words_at(opa, ob), z_voff);
-                tzz = load_elem<BF16, kNT>(words_at(ota, ob), z_voff);
+                pz = load_raw<BF16, LATE, kNT>(words_at(opa, ob), z_voff);
+                tzz = load_raw<BF16, LATE, kNT>(words_at(ota, ob), z_voff);
                 opa += PB;
                 ota += PB;
             }
