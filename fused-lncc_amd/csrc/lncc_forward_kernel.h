@@ -22,10 +22,10 @@
 // Bound: VALU issue. At k = 7 a plane of a 48 x 32 tile takes ~2150 cycles of a CU, of which its vector
 // instructions fill ~1550 per SIMD (additions and products issue in 2.3 cycles, DPP additions, max,
 // compares and selects in 4.2, the reciprocal in 8); the LDS is busy for ~800, HBM fetches each input
-// byte 1.005 times. At (2,16,128^3) fp32: 0.219 / 0.242 / 0.281 / 0.452 ms -> 0.150 / 0.171 / 0.191 /
-// 0.223 ms at k = 3 / 5 / 7 / 9 against the gradient kernel run without its adjoint, whose x pass
-// goes through LDS and whose tile carries the adjoint's halo (2.8 TB/s of 8 B per voxel at k = 7);
-// the map of 160x192x224 at k = 9 0.0556 -> 0.0378 ms. F is the longer role and has the lower wave
+// byte 1.005 times. At (2,16,128^3) fp32: 0.219 / 0.242 / 0.281 / 0.452 ms -> 0.150 / 0.164 / 0.179 /
+// 0.216 ms at k = 3 / 5 / 7 / 9 against the gradient kernel run without its adjoint, whose x pass
+// goes through LDS and whose tile carries the adjoint's halo (3.0 TB/s of 8 B per voxel at k = 7);
+// the map of 160x192x224 at k = 9 0.0556 -> 0.0356 ms. F is the longer role and has the lower wave
 // indices, which the SIMDs serve first (Y first: 9% slower at k = 7).
 #pragma once
 #include "lncc_common.h"
@@ -122,11 +122,21 @@ struct Pieces {
     }
 };
 
-// Tile -> volume, first input column, first output row.
-template <class G>
-__device__ __forceinline__ void tile_origin(const FusedArgs& a, uint32_t tile, int64_t& b, int& x0, int& y0) {
+// Tile -> volume, first input column, first output row. With WHOLE the tile that reaches past a row's
+// end starts up to NC - 1 columns earlier (not the first tile, which has none there), so that the last
+// columns of a lane are a row's last ones and no lane's columns are cut; `skip` is that number, by which
+// its own output columns start later.
+// Bound of a tile with cut lanes: its loads, NC times as many of 4 bytes each, up to half as long again
+// as the tiles beside it, for which a launch of one round waits. Loss at 160x192x224 k = 7 36.7 -> 25.2
+// us, 96^3 k = 9 12.7 -> 10.0, (2,16,128^3) k = 7 187 -> 178; map at 160x192x224 k = 7 33 -> 29,
+// (2,64,64^3) k = 7 152 -> 134; widths without cut lanes within 2%. bfloat16 loads one by one always.
+template <class G, int NC, bool WHOLE>
+__device__ __forceinline__ void tile_origin(const FusedArgs& a, uint32_t tile, int64_t& b, int& x0, int& y0, int& skip) {
     const uint32_t tx = tile % (uint32_t)a.ntx, t = tile / (uint32_t)a.ntx;
     x0 = (int)tx * G::ADV;
+    skip = 0;
+    if (WHOLE && tx > 0 && x0 + G::RW > a.dimW) skip = (NC - (a.dimW - x0) % NC) % NC;
+    x0 -= skip;
     y0 = (int)(t % (uint32_t)a.nty) * G::OY;
     b = (int64_t)(t / (uint32_t)a.nty);
 }
@@ -155,17 +165,17 @@ __global__ __launch_bounds__((FwdGeo<HH, NC>::LANES), 1) void lncc_forward_kerne
         uint32_t tile;
         while (pieces.next(tile, z0, z1)) {
         int64_t b;
-        int x0, y0;
-        tile_origin<G>(a, tile, b, x0, y0);
+        int x0, y0, skip;
+        tile_origin<G, NC, !BF16>(a, tile, b, x0, y0, skip);
         // F runs planes [tb, zend), whose windows are centred on [z0, z1), Y one step (PPB planes) later
         const int tb = z0 + HH, zend = z1 + HH, nsteps = (z1 - z0 + G::PPB - 1) / G::PPB + 1;
         const int gy = y0 - HH + iy, gx = x0 + NC * l;
         const bool row_in = gy >= 0 && gy < Hd;
         const uint32_t plane_bytes = (uint32_t)(HW * ELEM);
-        // float32 rows are one wide load per lane and field, except in a tile whose right edge cuts a
-        // lane's columns, where it would read the next row's: `inside` of them one by one
         const uint32_t at = (uint32_t)((gy * Wd + gx) * ELEM);
         const int inside = row_in ? Wd - gx : 0;
+        // float32 rows are one wide load per lane and field, except in a row's only tile where its right
+        // edge cuts a lane's columns and the load would read the next row's: `inside` of them one by one
         const bool wide = !BF16 && (x0 + G::RW <= Wd || (Wd - x0) % NC == 0);
         uint32_t voff[BF16 ? NC : 1];
         voff[0] = inside > 0 ? at : kOOB;
@@ -286,13 +296,13 @@ __global__ __launch_bounds__((FwdGeo<HH, NC>::LANES), 1) void lncc_forward_kerne
         uint32_t tile;
         while (pieces.next(tile, z0, z1)) {
         int64_t b;
-        int x0, y0;
-        tile_origin<G>(a, tile, b, x0, y0);
+        int x0, y0, skip;
+        tile_origin<G, NC, !BF16>(a, tile, b, x0, y0, skip);
         const int nsteps = (z1 - z0 + G::PPB - 1) / G::PPB + 1;
         const int gx = x0 + x, gy = y0 + seg * G::SY;
         // a column is this tile's if both neighbours' columns of its window were there, or are outside
         // the volume
-        const bool col = gx < Wd && (x0 == 0 || x >= HH) && (x < G::RW - HH || x0 + G::RW >= Wd);
+        const bool col = gx < Wd && (x0 == 0 || x >= HH + skip) && (x < G::RW - HH || x0 + G::RW >= Wd);
         float core[G::SY];
 #pragma unroll
         for (int i = 0; i < G::SY; ++i) core[i] = col && gy + i < Hd ? 1.f : 0.f;

@@ -42,6 +42,14 @@ def test_tile_edges(shape, k):
 
 
 @pytest.mark.parametrize("k", [3, 5, 7, 9])
+@pytest.mark.parametrize("width", [49, 50, 51, 52, 93, 94, 95, 96, 97, 121, 122, 123, 124, 125, 193])
+def test_last_tile_starts_early(width, k):
+    """Every remainder of a row's last tile by the lane's three or four columns, two to five tiles a row:
+    no column of the map left out or taken from the wrong tile, none counted twice in the loss."""
+    check(*wl.randn_pair((1, 2, 4, 9, width), 10 * width + k), k)
+
+
+@pytest.mark.parametrize("k", [3, 5, 7, 9])
 def test_bf16_odd_rows(k):
     check(*wl.randn_pair((1, 2, 6, 30, 51), k), k, torch.bfloat16)
 
