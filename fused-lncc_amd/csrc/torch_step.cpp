@@ -116,7 +116,10 @@ PyObject* step(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (nargs != 5 || !THPVariable_Check(args[0]) || !THPVariable_Check(args[1])) Py_RETURN_NONE;
     const long k = PyLong_AsLong(args[2]);
     const double dr = PyFloat_AsDouble(args[3]);
-    if (PyErr_Occurred()) return nullptr;
+    if (PyErr_Occurred()) {   // a kernel size past long: the Python path's refusal
+        PyErr_Clear();
+        Py_RETURN_NONE;
+    }
     const Tensor pred = THPVariable_Unpack(args[0]), target = THPVariable_Unpack(args[1]);
     const int code = dtype_code(pred);
     if (!pred.is_cuda() || pred.device() != target.device() || code < 0 || target.scalar_type() != pred.scalar_type() ||

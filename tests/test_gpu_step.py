@@ -142,7 +142,7 @@ def test_hooks_create_graph_and_streams(monkeypatch):
 def test_refusals_are_the_python_functions(monkeypatch):
     p, t = pair()
     for bad in (lambda: fused_lncc_loss(p.double(), t.double(), 7), lambda: fused_lncc_loss(p, t.bfloat16(), 7),
-                lambda: fused_lncc_loss(p.cpu(), t.cpu(), 7), lambda: fused_lncc_loss(p, t, 11),
+                lambda: fused_lncc_loss(p.cpu(), t.cpu(), 7), lambda: fused_lncc_loss(p, t, 11), lambda: fused_lncc_loss(p, t, 2 ** 70 + 1),
                 lambda: fused_lncc_loss(p, t.cpu(), 7), lambda: fused_lncc_loss(p[:, :0], t[:, :0], 7)):
         def f():
             with pytest.raises(RuntimeError) as e:
