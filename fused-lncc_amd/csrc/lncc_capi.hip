@@ -120,14 +120,16 @@ void try_forward(int64_t B, int64_t D, int64_t H_, int64_t W, int64_t gblocks, d
     }
 }
 
-ForwardPlan plan_forward(int64_t B, int64_t D, int64_t H, int64_t W, int halo, bool maps, int64_t gblocks) {
+ForwardPlan plan_forward(int64_t B, int64_t D, int64_t H, int64_t W, int halo, int64_t gblocks) {
     ForwardPlan f = {};
     double best = -1;
     // A plane of a 64-column tile (28 output rows) against one of a 48-column tile (32): 1.1x measured at
-    // k <= 5; at k = 7, where the four columns' rings fill the registers and a few spill, 1.13x for the
-    // loss ((2,64,64^3): 109 us in 64-column tiles, 117 in 48-column ones) and 1.4x for the maps
-    // (160x192x224: 38-41 and 34 us). At k = 9 they don't fit.
-    const double wide7 = maps ? 1.4 : 1.2;
+    // k <= 5 ((2,64,64^3) k = 3 loss: 76 us in 64-column tiles, 88 in 48-column ones; bfloat16 160x192x224
+    // k = 3 19.4 and 17.7). At k = 7, where the four columns' rings fill the registers and some spill,
+    // 1.2x: maps of (2,64,64^3) 120 and 134 us, bfloat16 143 and 157, of 3 volumes of 70x150x140 26.1 and
+    // 28.5; a loss term of these 22.9 and 24.0. On 160x192x224, where the plans cost the same, the map takes
+    // 28.4 and 29.3, the loss 26.0 and 24.5. At k = 9 they don't fit.
+    constexpr double wide7 = 1.2;
     switch (halo) {
         case 1: try_forward<1, 3>(B, D, H, W, gblocks, 1.0, f, best); try_forward<1, 4>(B, D, H, W, gblocks, 1.1, f, best); break;
         case 2: try_forward<2, 3>(B, D, H, W, gblocks, 1.0, f, best); try_forward<2, 4>(B, D, H, W, gblocks, 1.1, f, best); break;
@@ -199,7 +201,7 @@ hipError_t launch_fused(int halo, int mode, bool bf16, const fl::FusedArgs& a, c
 // The loss without a gradient, or the maps. `a` holds the arguments of the gradient plan g.
 hipError_t launch_forward(int64_t B, int halo, int mode, bool bf16, fl::FusedArgs a, const Plan& g, hipStream_t st) {
     if (g.small) return fl::launch_small(halo, mode, bf16, a, (uint32_t)g.nblocks, st);
-    const ForwardPlan f = plan_forward(B, a.dimD, a.dimH, a.dimW, halo, mode == fl::MODE_MAPS, g.nblocks);
+    const ForwardPlan f = plan_forward(B, a.dimD, a.dimH, a.dimW, halo, g.nblocks);
     a.ntx = f.ntx;
     a.nty = f.nty;
     a.nzc = f.nzc;
