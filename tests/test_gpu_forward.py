@@ -19,20 +19,22 @@ SHAPES = [
 ]
 
 
-def check(p, t, k, dtype=torch.float32):
+def check(p, t, k, dtype=torch.float32, dr=1e-5):
     """Loss and map against the float64 oracle, bounded by RATIO times the error of the reference's own
     float32 arithmetic on the same values (the loss is their mean: at most its largest error), or by
     float32's rounding of the result."""
     pd, td = p.to(dtype).to(DEV), t.to(dtype).to(DEV)
     pn, tn = pd.float().cpu().numpy(), td.float().cpu().numpy()
     with torch.no_grad():
-        loss = fused_lncc_loss(pd, td, k).item()
-    m = lncc_map(pd, td, k).double().cpu().numpy()
-    l64, _, maps = O.lncc(pn, tn, k, 1e-5, grad=True, maps=True)
-    l32, _, m32 = O.lncc_ref32(pn, tn, k, 1e-5, grad=True, ncc_map=True)
+        loss = fused_lncc_loss(pd, td, k, dr).item()
+    m = lncc_map(pd, td, k, dr).double().cpu().numpy()
+    l64, _, maps = O.lncc(pn, tn, k, dr, grad=True, maps=True)
+    l32, _, m32 = O.lncc_ref32(pn, tn, k, dr, grad=True, ncc_map=True)
     err32 = np.abs(m32.astype(np.float64) - maps["ncc"])
     assert np.abs(m - maps["ncc"]).max() <= max(RATIO * err32.max(), 1e-5)
-    assert abs(loss - l64) <= max(RATIO * max(abs(l32 - l64), err32.mean()), 2e-7)
+    bound = max(RATIO * max(abs(l32 - l64), err32.mean()), 2e-7)
+    assert abs(loss - l64) <= bound
+    return l64, bound
 
 
 @pytest.mark.parametrize("k", [3, 5, 7, 9])
@@ -88,3 +90,17 @@ def test_nan_reaches_the_loss(where):
     p[(0, 0) + where] = float("nan")
     with torch.no_grad():
         assert torch.isnan(fused_lncc_loss(p.to(DEV), t.to(DEV), 7)).item()
+
+
+@pytest.mark.parametrize("dr", [0.0, 1e-20])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("k", [3, 5, 7, 9])
+@pytest.mark.parametrize("shape", [(1, 2, 9, 75, 40), (1, 1, 17, 32, 32), (1, 1, 5, 96, 96)])
+def test_windows_past_the_volume_do_not_reach_the_loss(shape, k, dtype, dr):
+    """Tiles reach past the volume by more than h rows or columns, where a window is all zeros: at a
+    smooth_dr of 0 (or one whose square has no float32 reciprocal) its ncc is 0 * inf, which counts in
+    no loss. With and without a gradient the loss is the oracle's."""
+    p, t = wl.randn_pair(shape, 7 * k + shape[3])
+    l64, bound = check(p, t, k, dtype, dr)
+    with_grad = fused_lncc_loss(p.to(dtype).to(DEV).requires_grad_(True), t.to(dtype).to(DEV), k, dr).item()
+    assert abs(with_grad - l64) <= bound
