@@ -329,6 +329,36 @@ def test_first_use_builds_missing_library(tmp_path):
     assert out.stdout.strip() == f"loaded {pkg / 'fused_lncc' / 'libfused_lncc_hip.so'} True"
 
 
+@pytest.mark.parametrize("missing", ["compiler", "headers", "torch"])
+def test_library_is_built_without_the_extension(tmp_path, missing):
+    """The library needs hipcc only: where the eager-step extension cannot be built, build.py installs
+    the library, says why the extension is not there, leaves none of an earlier build, and fails only
+    under --require-step. (A stand-in for hipcc that writes its output file: what is tested is the order.)"""
+    import subprocess
+    import sys
+    pkg = _package_copy(tmp_path)
+    hipcc = tmp_path / "hipcc"
+    hipcc.write_text('#!/bin/sh\nwhile [ "$1" != -o ]; do shift; done\necho built > "$2"\n')
+    hipcc.chmod(0o755)
+    env = dict(os.environ, HIPCC=str(hipcc))
+    if missing == "compiler":
+        env["CXX"] = "/nonexistent/c++"
+    elif missing == "headers":
+        env["CXX"] = "false"   # every compilation fails
+    else:
+        (tmp_path / "torch.py").write_text("raise ImportError('no torch here')\n")
+        env["PYTHONPATH"] = str(tmp_path)
+    lib, step = (pkg / "fused_lncc" / n for n in ("libfused_lncc_hip.so", "_step.so"))
+    for require in (False, True):
+        step.write_text("of an earlier build")
+        r = subprocess.run([sys.executable, str(pkg / "build.py")] + ["--require-step"] * require, capture_output=True,
+                           text=True, env=env, timeout=300)
+        assert (r.returncode != 0) == require, r.stderr
+        assert lib.read_text().strip() == "built" and not step.exists()
+        assert "building _step.so failed" in r.stderr
+        lib.unlink()
+
+
 def test_bench_refuses_more_than_one_gpu():
     """bench.py measures one GPU; --gpus N > 1 exits with status 2 and says so, before touching a
     device."""
