@@ -1,9 +1,9 @@
 """Build libfused_lncc_hip.so for gfx950 in-tree: one hipcc job per translation unit, then link; and
-_step.so, the eager step as a torch extension (host code only), with the host compiler.
+_step, the eager step as a torch extension (host code only), with the host compiler.
 
 Usage: ``python fused-lncc_amd/build.py [--jobs N] [--require-step]``. Both land next to the Python
 package (``fused-lncc_amd/fused_lncc/``), objects under ``fused-lncc_amd/_build/``. The library needs
-hipcc only. _step.so is optional (without it the Python autograd function does the same): where it
+hipcc only. _step is optional (without it the Python autograd function does the same): where it
 cannot be built, for want of torch, its headers or a host compiler, the reason goes to stderr and the
 build succeeds; with ``--require-step`` it then fails, after the library is in place.
 """
@@ -12,12 +12,13 @@ import concurrent.futures as cf
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "fused_lncc", "libfused_lncc_hip.so")
-STEP = os.path.join(HERE, "fused_lncc", "_step.so")
+STEP = os.path.join(HERE, "fused_lncc", "_step" + sysconfig.get_config_var("EXT_SUFFIX"))   # for this interpreter
 ARCH = os.environ.get("FUSED_LNCC_ARCH", "gfx950")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
@@ -39,15 +40,15 @@ def _compile(src):
 
 
 def _build_step():
-    """_step.so (csrc/torch_step.cpp) against the installed torch's headers and libraries. The torch
-    libraries are found where torch loaded them from when the module is imported."""
-    import sysconfig
+    """The extension (csrc/torch_step.cpp) against the installed torch's headers and libraries, which it
+    names in itself. The torch libraries are found where torch loaded them from when it is imported."""
     import torch
     root = os.path.dirname(torch.__file__)
     inc = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
            os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"), sysconfig.get_paths()["include"]]
     cmd = ([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
-            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__"]
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            f'-DFL_TORCH="{torch.__version__} {torch.version.git_version}"', "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__"]
            + [a for i in inc for a in ("-isystem", i)] + [os.path.join(CSRC, "torch_step.cpp"), "-o", STEP + ".tmp"]
            + ["-L" + os.path.join(root, "lib"), "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", "-lc10_hip"])
     r = subprocess.run(cmd, capture_output=True, text=True)
@@ -75,17 +76,17 @@ def build(jobs=None, verbose=True, require_step=False):
     except Exception as e:   # a torch that does not load or is laid out otherwise, no compiler, a failed compilation
         if os.path.exists(STEP):   # of an earlier build
             os.remove(STEP)
-        msg = f"building _step.so failed ({type(e).__name__}: {e})"
+        msg = f"building _step failed ({type(e).__name__}: {e})"
         if require_step:
             raise RuntimeError(msg) from e
-        print(f"{msg}\nThe library is built; without _step.so the Python autograd function is used.", file=sys.stderr)
+        print(f"{msg}\nThe library is built; without _step the Python autograd function is used.", file=sys.stderr)
     return LIB
 
 
 if __name__ == "__main__":
     ap = argparse.ArgumentParser()
     ap.add_argument("--jobs", type=int, default=None)
-    ap.add_argument("--require-step", action="store_true", help="fail where _step.so cannot be built")
+    ap.add_argument("--require-step", action="store_true", help="fail where _step cannot be built")
     a = ap.parse_args()
     try:
         build(a.jobs, require_step=a.require_step)

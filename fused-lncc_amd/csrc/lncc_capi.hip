@@ -278,7 +278,7 @@ int scratch_on_current_device(double** out) {
 
 extern "C" {
 
-int fl_version(void) { return (0 << 16) | (2 << 8) | 0; }
+int fl_version(void) { return FL_VERSION; }
 
 int fl_test_set_dchunk(int planes) {
     if (planes < 0) return fail(FL_E_SHAPE, "fl_test_set_dchunk: negative chunk length");

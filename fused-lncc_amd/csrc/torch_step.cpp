@@ -167,4 +167,13 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_step", nullptr, -1, methods, null
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__step(void) { return PyModule_Create(&module); }
+// TORCH: the torch that this was compiled against, whose object layouts it uses; FL_VERSION: the C ABI's
+// version whose signatures it calls. The loader compares both before init().
+PyMODINIT_FUNC PyInit__step(void) {
+    PyObject* m = PyModule_Create(&module);
+    if (m && (PyModule_AddStringConstant(m, "TORCH", FL_TORCH) < 0 || PyModule_AddIntConstant(m, "FL_VERSION", FL_VERSION) < 0)) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}

@@ -111,12 +111,18 @@ _step = None   # the extension's step(), False where it cannot be loaded
 
 def eager_step():
     """step() of the eager-step extension, bound to the loaded library, or None where the extension is
-    not there (or was built for another torch): the Python autograd function then does the same."""
+    not there or was built for another torch or library: the Python autograd function then does the same."""
     global _step
     if _step is None:
         lib = load()
         try:
+            import torch
             from . import _step as ext_module
+            # another torch's symbols may resolve although its objects are laid out otherwise
+            built = getattr(ext_module, "TORCH", None), getattr(ext_module, "FL_VERSION", None)
+            here = f"{torch.__version__} {torch.version.git_version}", lib.fl_version()
+            if built != here:
+                raise ImportError(f"built for torch and library version {built}, these are {here}")
             ext_module.init(*[ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in _STEP_API])
             _step = ext_module.step
         except ImportError as e:

@@ -32,7 +32,9 @@ enum fl_status {
     FL_E_DEVICE = -6     /* HIP runtime or launch error */
 };
 
-/* Library version, (major << 16) | (minor << 8) | patch. */
+/* Library version, (major << 16) | (minor << 8) | patch; fl_version() gives the loaded library's, FL_VERSION the
+ * one these declarations belong to. A changed declaration changes it. */
+#define FL_VERSION ((0 << 16) | (2 << 8) | 0)
 int fl_version(void);
 
 /* Message of the last failing call on this thread ("" if none). The text is owned by the library

@@ -336,6 +336,7 @@ def test_library_is_built_without_the_extension(tmp_path, missing):
     under --require-step. (A stand-in for hipcc that writes its output file: what is tested is the order.)"""
     import subprocess
     import sys
+    import sysconfig
     pkg = _package_copy(tmp_path)
     hipcc = tmp_path / "hipcc"
     hipcc.write_text('#!/bin/sh\nwhile [ "$1" != -o ]; do shift; done\necho built > "$2"\n')
@@ -348,15 +349,32 @@ def test_library_is_built_without_the_extension(tmp_path, missing):
     else:
         (tmp_path / "torch.py").write_text("raise ImportError('no torch here')\n")
         env["PYTHONPATH"] = str(tmp_path)
-    lib, step = (pkg / "fused_lncc" / n for n in ("libfused_lncc_hip.so", "_step.so"))
+    lib, step = (pkg / "fused_lncc" / n for n in ("libfused_lncc_hip.so", "_step" + sysconfig.get_config_var("EXT_SUFFIX")))
     for require in (False, True):
         step.write_text("of an earlier build")
         r = subprocess.run([sys.executable, str(pkg / "build.py")] + ["--require-step"] * require, capture_output=True,
                            text=True, env=env, timeout=300)
         assert (r.returncode != 0) == require, r.stderr
         assert lib.read_text().strip() == "built" and not step.exists()
-        assert "building _step.so failed" in r.stderr
+        assert "building _step failed" in r.stderr
         lib.unlink()
+
+
+@pytest.mark.parametrize("other", [None, ("TORCH", "2.9.1+rocm6.4 0123"), ("FL_VERSION", 1)])
+def test_extension_of_another_torch_or_library_is_not_used(monkeypatch, capsys, other):
+    """The eager-step extension works on torch's objects as its headers lay them out and calls the C ABI
+    as they declare it: one built for another torch or another version of the library is not initialised,
+    and the Python autograd function is used."""
+    from fused_lncc import _step
+    monkeypatch.setattr(_lib, "_step", None)
+    if other is None:
+        assert _lib.eager_step() is _step.step
+        return
+    monkeypatch.setattr(_step, *other, raising=False)
+    monkeypatch.setattr(_step, "init", lambda *a: pytest.fail("initialised"))
+    assert _lib.eager_step() is None
+    assert "the eager-step extension is not used" in capsys.readouterr().err
+    assert _lib.eager_step() is None and capsys.readouterr().err == ""   # said once
 
 
 def test_bench_refuses_more_than_one_gpu():
