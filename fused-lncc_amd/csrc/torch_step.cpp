@@ -6,7 +6,8 @@
 // Python node makes the autograd thread take the interpreter lock.
 //
 // A Python extension module without a link to the HIP library: init() receives the addresses of the C
-// ABI's functions from the loader, so that both paths use the one library that it loaded.
+// ABI's functions and the package's error class from the loader, so that both paths use the one library
+// that it loaded and raise the same errors.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #include <torch/csrc/autograd/custom_function.h>
@@ -32,13 +33,28 @@ struct Api {
     decltype(&fl_lncc_loss_grad_pt) loss_grad_pt;
     decltype(&fl_scale_grad) scale_grad;
     decltype(&fl_last_error) last_error;
+    PyObject* error;   // FusedLNCCError(code, message)
 } api;
 
 int dtype_code(const Tensor& t) {
     return t.scalar_type() == at::kFloat ? FL_F32 : t.scalar_type() == at::kBFloat16 ? FL_BF16 : -1;
 }
 
-void check(int rc) { TORCH_CHECK(rc == FL_OK, api.last_error()); }
+// The library's refusal as the Python path raises it; called with or without the interpreter lock, on the
+// caller's or on an autograd thread (which hands a Python error on to the one that waits for it).
+void check(int rc) {
+    if (rc == FL_OK) return;
+    const std::string msg = api.last_error();
+    pybind11::gil_scoped_acquire gil;
+    PyObject* text = PyUnicode_DecodeUTF8(msg.data(), (Py_ssize_t)msg.size(), "replace");
+    PyObject* e = text ? PyObject_CallFunction(api.error, "iO", rc, text) : nullptr;
+    if (e) PyErr_SetObject(api.error, e);
+    Py_XDECREF(e);
+    Py_XDECREF(text);
+    python_error err;
+    err.persist();
+    throw err;
+}
 
 void* stream_of(const Tensor& t) {
     return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream();
@@ -148,7 +164,11 @@ PyObject* step(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 
 PyObject* init(PyObject*, PyObject* args) {
     unsigned long long a[6];
-    if (!PyArg_ParseTuple(args, "KKKKKK", &a[0], &a[1], &a[2], &a[3], &a[4], &a[5])) return nullptr;
+    PyObject* error;
+    if (!PyArg_ParseTuple(args, "KKKKKKO", &a[0], &a[1], &a[2], &a[3], &a[4], &a[5], &error)) return nullptr;
+    Py_INCREF(error);
+    Py_XDECREF(api.error);
+    api.error = error;
     api.validate = reinterpret_cast<decltype(api.validate)>(a[0]);
     api.workspace_bytes = reinterpret_cast<decltype(api.workspace_bytes)>(a[1]);
     api.loss_grad = reinterpret_cast<decltype(api.loss_grad)>(a[2]);

@@ -123,7 +123,7 @@ def eager_step():
             here = f"{torch.__version__} {torch.version.git_version}", lib.fl_version()
             if built != here:
                 raise ImportError(f"built for torch and library version {built}, these are {here}")
-            ext_module.init(*[ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in _STEP_API])
+            ext_module.init(*[ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in _STEP_API], FusedLNCCError)
             _step = ext_module.step
         except ImportError as e:
             print(f"fused_lncc: the eager-step extension is not used ({e}); run `python fused-lncc_amd/build.py`",

@@ -152,6 +152,45 @@ def test_refusals_are_the_python_functions(monkeypatch):
         assert got == want
 
 
+def error_of(f):
+    with pytest.raises(RuntimeError) as e:
+        f()
+    return type(e.value), getattr(e.value, "code", None), str(e.value)
+
+
+def test_library_errors_are_the_python_functions(monkeypatch):
+    """What the library itself refuses once the arguments are valid (here, on the host, a forced chunk
+    length that makes more workgroups than one launch holds) is a FusedLNCCError with its code."""
+    x = torch.zeros(2100000, 1, 2, 1, 1, device=DEV)
+    with _lib.dchunk(1):
+        got, want = both(monkeypatch, lambda: error_of(lambda: fused_lncc_loss(x, x, 3)))
+    assert got == want and got[0] is _lib.FusedLNCCError and got[1] == _lib.FL_E_NULL
+
+
+def test_library_errors_in_backward_are_the_python_functions(monkeypatch):
+    """A device error that the backward's library call reports, on the autograd thread, reaches the
+    caller as a FusedLNCCError with its code. (A stand-in for fl_scale_grad that launches nothing.)"""
+    import ctypes
+    from fused_lncc import _step
+    lib = _lib.load()
+    real = {n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in _lib._STEP_API}
+    fails = ctypes.CFUNCTYPE(ctypes.c_int, *_lib.SIGNATURES["fl_scale_grad"][1])(lambda *a: _lib.FL_E_DEVICE)
+
+    def f():
+        p, t = pair()
+        loss = fused_lncc_loss(p.requires_grad_(True), t, 7)
+        return error_of(loss.backward)
+    assert _lib.eager_step() is not None
+    try:
+        _step.init(*{**real, "fl_scale_grad": ctypes.cast(fails, ctypes.c_void_p).value}.values(), _lib.FusedLNCCError)
+        with monkeypatch.context() as m:
+            m.setattr(lib, "fl_scale_grad", fails)
+            got, want = both(monkeypatch, f)
+    finally:
+        _step.init(*real.values(), _lib.FusedLNCCError)
+    assert got[:2] == want[:2] == (_lib.FusedLNCCError, _lib.FL_E_DEVICE)
+
+
 def test_watched_calls_keep_the_python_function(monkeypatch):
     calls = []
     step = _lib.eager_step()
