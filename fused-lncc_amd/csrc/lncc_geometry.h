@@ -152,6 +152,7 @@ struct FwdGeo {
     static constexpr int PPB = H == 4 ? 2 : 1;
     static constexpr int XP = fits(PPB, rup64(XP0)) ? rup64(XP0) : XP0;
     static constexpr int PLANE = 5 * XP, BUF = PPB * PLANE;
+    static constexpr int LDS_BYTES = 2 * BUF * 4 + NYW * 8;   // and the Y waves' partials of the loss
     static_assert(NYW * 64 == RW * YSEG && LANES <= 1024 && XS % 4 == 2 && fits(PPB, XP), "lanes");
 };
 

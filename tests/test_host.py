@@ -108,6 +108,14 @@ def test_lds_bytes():
     assert lib.fl_lds_bytes(8, _lib.FL_F32) == 0 and lib.fl_lds_bytes(7, 5) == 0
 
 
+def test_lds_bytes_is_the_largest_of_all_kernels():
+    """Kernel by kernel what the compiler reports: the small-volume kernel 131200 B, the gradient kernel
+    with both gradients 125184 / 147264 / 161184 / 150784 B, the forward-only kernel's larger tile 76856 /
+    87096 / 87096 / 161328 B at k = 3 / 5 / 7 / 9."""
+    lib = _lib.load()
+    assert [lib.fl_lds_bytes(k, _lib.FL_F32) for k in (3, 5, 7, 9)] == [131200, 147264, 161184, 161328]
+
+
 def test_shape_limits_without_overflow():
     lib = _lib.load()
     # H*W*4 would overflow int64: refused by the per-dimension bound first
