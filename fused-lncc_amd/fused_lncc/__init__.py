@@ -222,7 +222,7 @@ def fused_lncc_loss(pred, target, kernel_size=7, smooth_dr=1e-5, *, target_grad=
     (2,16,128^3) k=7); volumes of at most 16^3 take a second pass with pred and target swapped."""
     assert pred.dim() == 5 and pred.shape == target.shape, "expect matching (N,C,D,H,W)"
     assert kernel_size % 2 == 1, "kernel_size must be odd"
-    if type(pred) in _PLAIN and type(target) in _PLAIN and not _watched():
+    if type(pred) in _PLAIN and type(target) in _PLAIN and pred.is_cuda and not _watched():
         step = _lib.eager_step()
         if step is not None:
             loss = step(pred, target, int(kernel_size), float(smooth_dr), bool(target_grad))

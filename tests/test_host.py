@@ -304,6 +304,27 @@ def test_missing_library_fails_loudly():
     assert "ImportError:" in out.stdout and "no CPU fallback" in out.stdout
 
 
+def test_host_tensors_are_refused_without_the_library():
+    """CPU tensors are refused for what they are before the library is looked for (or built)."""
+    import subprocess
+    import sys
+    code = ("import torch\n"
+            "import fused_lncc._lib as L\n"
+            "L.LIB_PATH = '/nonexistent/libfused_lncc_hip.so'\n"
+            "from fused_lncc import fused_lncc_loss\n"
+            "p = torch.randn(1, 1, 8, 8, 8)\n"
+            "for x in (p, p.double(), p.requires_grad_(True)):\n"
+            "    try:\n"
+            "        fused_lncc_loss(x, x.detach(), 7)\n"
+            "    except RuntimeError as e:\n"
+            "        print('RuntimeError:', e)\n")
+    env = dict(os.environ, PYTHONPATH=os.path.join(ROOT, "fused-lncc_amd"))
+    out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, env=env, timeout=300)
+    assert out.returncode == 0, out.stderr
+    lines = out.stdout.strip().splitlines()
+    assert len(lines) == 3 and "GPU tensor" in lines[0] and "float32 or bfloat16" in lines[1] and "GPU tensor" in lines[2]
+
+
 def _package_copy(tmp_path):
     """The package, its build script and HIP sources, and the C-ABI header they include, copied
     without any built file."""
