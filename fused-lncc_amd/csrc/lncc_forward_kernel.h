@@ -159,8 +159,8 @@ __global__ __launch_bounds__((FwdGeo<HH, NC>::LANES), 1) void lncc_forward_kerne
 
     if (wave_id < G::NFW) {
         // ---------------- F waves ----------------
-        const int l = tid & 15, iy = min(tid >> 4, G::IY - 1);   // rows past the last repeat it
-        float* const xs = Xs + l * G::XS + iy;   // row j * 16 + l of field q: + q * XP + j * 16 XS
+        int l, iy;
+        float* const xs = Xs + fwd_f_lane<G>(tid, l, iy);
         int z0, z1;
         uint32_t tile;
         while (pieces.next(tile, z0, z1)) {
@@ -168,11 +168,11 @@ __global__ __launch_bounds__((FwdGeo<HH, NC>::LANES), 1) void lncc_forward_kerne
         int x0, y0, skip;
         tile_origin<G, NC, !BF16>(a, tile, b, x0, y0, skip);
         // F runs planes [tb, zend), whose windows are centred on [z0, z1), Y one step (PPB planes) later
-        const int tb = z0 + HH, zend = z1 + HH, nsteps = (z1 - z0 + G::PPB - 1) / G::PPB + 1;
+        const int tb = z0 + HH, zend = z1 + HH, nsteps = fwd_steps<G>(z1 - z0);
         const int gy = y0 - HH + iy, gx = x0 + NC * l;
         const bool row_in = gy >= 0 && gy < Hd;
         const uint32_t plane_bytes = (uint32_t)(HW * ELEM);
-        const uint32_t at = (uint32_t)((gy * Wd + gx) * ELEM);
+        const uint32_t at = ((uint32_t)gy * (uint32_t)Wd + (uint32_t)gx) * ELEM;   // used only inside the volume
         const int inside = row_in ? Wd - gx : 0;
         // float32 rows are one wide load per lane and field, except in a row's only tile where its right
         // edge cuts a lane's columns and the load would read the next row's: `inside` of them one by one
@@ -237,7 +237,7 @@ __global__ __launch_bounds__((FwdGeo<HH, NC>::LANES), 1) void lncc_forward_kerne
         if constexpr (CH) form_chain();
         // The march is unrolled by 2 k: the ring slot is the plane's position in its block of k, the
         // buffers alternate with its parity.
-        uint32_t buf = 0;   // LDS offset of the buffer being written
+        uint32_t buf = G::F_BUF0;   // LDS offset of the buffer being written
         for (int base = tb; base < tb + nsteps * G::PPB; base += 2 * K) {
             static_for<0, 2 * K>([&](auto uc) __attribute__((always_inline)) {
                 constexpr int u = decltype(uc)::value, r = u % K, par = u % 2;
@@ -277,17 +277,15 @@ __global__ __launch_bounds__((FwdGeo<HH, NC>::LANES), 1) void lncc_forward_kerne
                 fetch(zi + 2, p, t);
                 if constexpr (u % G::PPB == G::PPB - 1) {
                     __syncthreads();
-                    buf = G::BUF - buf;
+                    buf = fwd_other<G>(buf);
                 }
             });
         }
         }
     } else {
         // ---------------- Y waves ----------------
-        const int yl = tid - 64 * G::NFW;
-        const int seg = yl / G::RW, xr = yl - seg * G::RW;
-        const int x = NC * (xr & 15) + (xr >> 4);
-        const float* const xs = Xs + xr * G::XS + seg * G::SY;
+        int seg, x;
+        const float* const xs = Xs + fwd_y_lane<G>(tid - 64 * G::NFW, seg, x);
         float ndr = a.ndr;
         asm("" : "+v"(ndr));   // in a vector register: an addition with a scalar operand takes twice the cycles
         double loss_acc = 0.0;
@@ -298,7 +296,7 @@ __global__ __launch_bounds__((FwdGeo<HH, NC>::LANES), 1) void lncc_forward_kerne
         int64_t b;
         int x0, y0, skip;
         tile_origin<G, NC, !BF16>(a, tile, b, x0, y0, skip);
-        const int nsteps = (z1 - z0 + G::PPB - 1) / G::PPB + 1;
+        const int nsteps = fwd_steps<G>(z1 - z0);
         const int gx = x0 + x, gy = y0 + seg * G::SY;
         // a column is this tile's if both neighbours' columns of its window were there, or are outside
         // the volume
@@ -306,7 +304,7 @@ __global__ __launch_bounds__((FwdGeo<HH, NC>::LANES), 1) void lncc_forward_kerne
         bool core[G::SY];
 #pragma unroll
         for (int i = 0; i < G::SY; ++i) core[i] = col && gy + i < Hd;
-        uint32_t buf = G::BUF;   // the buffer written one step ago
+        uint32_t buf = G::Y_BUF0;   // the buffer written one step ago
         for (int st = 0; st < nsteps; ++st) {
             // the planes that this step's sums are centred on: zc .. zc + PPB - 1
             const int zc = z0 + (st - 1) * G::PPB;
@@ -363,7 +361,7 @@ __global__ __launch_bounds__((FwdGeo<HH, NC>::LANES), 1) void lncc_forward_kerne
                 }
             }
             __syncthreads();
-            buf = G::BUF - buf;
+            buf = fwd_other<G>(buf);
         }
         }
         if constexpr (MODE != MODE_MAPS) {

@@ -124,39 +124,24 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
     for (int j = 0; j < J; ++j) {
         int ix, iy;
         voff[j] = kOOB;
-        // a lane past the last column repeats it (with FPAIR it writes zeros into the padding): the
-        // same values to the same address, so that no store needs a lane mask
-        const int c = G::FPAIR ? tid + j * NT : min(tid + j * NT, G::NIN - 1);
-        if (f_column<G>(c, ix, iy, zaddr[j])) {
+        if (f_column<G>(f_lane<G>(tid + j * NT), ix, iy, zaddr[j])) {
             const int gx = x0 - 2 * HH + ix, gy = y0 - 2 * HH + iy;
             if (gx >= 0 && gx < Wd && gy >= 0 && gy < Hd) voff[j] = (uint32_t)((gy * Wd + gx) * ELEM);
         }
     }
     if constexpr (G::FPAIR) zaddr[1] = zaddr[0] + NT;
-    const bool f_col1 = G::FPAIR || (HH == 4 && DUAL) || wave_id * 64 + NT < G::NIN;   // this wave has second columns
+    const bool f_col1 = f_wave1<G>(wave_id);   // this wave has second columns
     // Y items on lanes [0, YITEMS) (y-sums in P0, ncc arithmetic in P1), X and AYs units in P1,
     // AX units in P0 (lncc_geometry.h); offsets into the source and destination buffers
     // (a lane has at most one unit of X and AYs, so the two share one pair of offsets; with five
     // adjoint fields the AYs units sit on Y lanes)
-    // The roles are whole waves (ROLE below), so that a stage is entered through one scalar compare
-    // and branch; a lane past the last unit of a role's last wave repeats that unit (the same values
-    // to the same addresses).
-    const bool wave_y = wave_id < G::NYW;
-    const bool wave_x = !wave_y && wave_id < G::NYW + G::NXW;
-    const bool wave_b = wave_id >= G::BL0 / 64 ? wave_id < G::BL0 / 64 + cdiv(G::BOWN, 64)
-                                               : wave_id < cdiv(G::UB - G::BOWN, 64);
-    bool wave_a = false;
-#pragma unroll
-    for (int sl = 0; sl < G::NAW; ++sl) wave_a = wave_a || wave_id == ax_wave<G>(sl);
+    // The roles are whole waves, so that a stage is entered through one scalar compare and branch.
+    const bool wave_y = y_wave<G>(wave_id), wave_x = x_wave<G>(wave_id), wave_b = ays_wave<G>(wave_id),
+               wave_a = a_wave<G>(wave_id);
     int u_src = 0, u_dst = 0, a_src, a_dst;
-    x_unit<G>(min(tid, G::XL0 + G::UX - 1), u_src, u_dst);
-    {
-        // the lane of the last AX unit, for the lanes past it in its wave
-        constexpr int LAST = ax_wave<G>(G::NAW - 1) * 64 + (G::UA - 1) % 64;
-        ax_unit<G>((tid >> 6) == ax_wave<G>(G::NAW - 1) ? min(tid, LAST) : tid, a_src, a_dst);
-    }
-    if (wave_b)
-        ays_unit<G>(tid >= G::BL0 ? min(tid, G::BL0 + G::BOWN - 1) : min(tid, G::UB - G::BOWN - 1), u_src, u_dst);
+    x_unit<G>(x_lane<G>(tid), u_src, u_dst);
+    ax_unit<G>(ax_lane<G>(tid), a_src, a_dst);
+    if (wave_b) ays_unit<G>(ays_lane<G>(tid), u_src, u_dst);
     int y_seg = 0, y_ax = 0;  // rows seg of AX positions
     // the Y item's offsets into Xs and Gs. At k = 7 they take the registers of the X / AYs unit
     // offsets (a Y lane has no such unit), which with three of Y's rows in flight across F is
@@ -165,7 +150,7 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
     constexpr bool Y_SHARE = HH == 3 && !DUAL;
     int y_xs = 0, y_gs0 = 0;
     if (wave_y) {
-        const int item = min(tid, G::YITEMS - 1);
+        const int item = y_lane<G>(tid);
         y_item<G>(item, y_seg, y_ax);
         if constexpr (Y_SHARE)
             y_offsets<G>(item, u_src, u_dst);

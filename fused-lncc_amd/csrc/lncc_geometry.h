@@ -1,6 +1,7 @@
-// Tile geometry and per-lane work maps of the fused LNCC kernel. Plain C++ (no HIP builtins):
-// the kernel takes every LDS offset it uses from these functions, and the host-side model of the
-// kernel's LDS accesses (tests/lds_model.cpp) enumerates the same functions for every lane.
+// Tile geometry and per-lane work maps of the LNCC kernels. Plain C++ (no HIP builtins): the kernels
+// take their roles and every LDS offset they use from these functions, and the host-side models of
+// their LDS accesses (tests/lds_model.cpp, forward_lds_model.cpp, small_lds_model.cpp) enumerate the
+// same functions for every lane.
 #pragma once
 
 #if defined(__HIPCC__)
@@ -135,6 +136,7 @@ struct Geo {
 // ---- the forward-only kernel (lncc_forward_kernel.h): NC columns per F lane, 16 lanes per row.
 template <int H, int NC>
 struct FwdGeo {
+    static constexpr int HALO = H, COLS = NC;
     static constexpr int SY = 4;                                    // output rows per Y lane
     static constexpr int RW = 16 * NC, ADV = RW - 2 * H;            // tile width, distance of tiles
     static constexpr int YSEG = NC == 3 ? 8 : 7, OY = YSEG * SY;    // output rows of a tile
@@ -154,7 +156,37 @@ struct FwdGeo {
     static constexpr int PLANE = 5 * XP, BUF = PPB * PLANE;
     static constexpr int LDS_BYTES = 2 * BUF * 4 + NYW * 8;   // and the Y waves' partials of the loss
     static_assert(NYW * 64 == RW * YSEG && LANES <= 1024 && XS % 4 == 2 && fits(PPB, XP), "lanes");
+    // A march over n output planes takes fwd_steps(n) steps, one barrier each: in step s F writes the planes
+    // s * PPB .. of them into one buffer, Y reads those of step s - 1 from the other. Offsets of the buffers
+    // of a march's first step (Y reads nothing there), which change place after every step.
+    static constexpr int F_BUF0 = 0, Y_BUF0 = BUF;
 };
+template <class G>
+FL_HD constexpr int fwd_other(int buf) {
+    return G::BUF - buf;
+}
+template <class G>
+FL_HD constexpr int fwd_steps(int planes) {
+    return (planes + G::PPB - 1) / G::PPB + 1;
+}
+// F lane tid: lane l of its row iy of the input region (lanes past the last row repeat it: the same values
+// to the same addresses); it writes column NC l + j of field q at the returned offset + q * XP + j * 16 * XS
+// of a plane.
+template <class G>
+FL_HD inline int fwd_f_lane(int tid, int& l, int& iy) {
+    l = tid & 15;
+    iy = tid >> 4 < G::IY - 1 ? tid >> 4 : G::IY - 1;
+    return l * G::XS + iy;
+}
+// Y lane yl (from the first Y wave on): column x of the tile and rows seg * SY .. of its output rows; it
+// reads SY + 2h input rows from the returned offset + q * XP of a plane.
+template <class G>
+FL_HD inline int fwd_y_lane(int yl, int& seg, int& x) {
+    seg = yl / G::RW;
+    const int xr = yl - seg * G::RW;
+    x = G::COLS * (xr & 15) + (xr >> 4);
+    return xr * G::XS + seg * G::SY;
+}
 
 // ---- the small-volume kernel (lncc_small.hip): one workgroup of kSmallLanes lanes per volume
 // whose D, H, W are all at most kSmallEdge, the volume zero-padded to kSmallEdge^3 in LDS. Lanes
@@ -193,6 +225,45 @@ FL_HD inline void split32(int idx, int n_rows, int& row, int& pos) {
     }
 }
 
+// The plane-marching kernel's roles are whole waves: which waves take Y items (y-sums in P0, ncc
+// arithmetic in P1), X units, AYs units (P1; with five adjoint fields some of them on Y waves) and AX
+// units (P0), and which have second F columns. A lane past the last unit of a role's last wave repeats
+// that unit, the same values to the same addresses, so that no stage needs a lane mask: *_lane gives the
+// lane whose unit a lane of the role takes (f_lane the input column).
+template <class G>
+FL_HD constexpr bool y_wave(int wave) {
+    return wave < G::NYW;
+}
+template <class G>
+FL_HD constexpr bool x_wave(int wave) {
+    return !y_wave<G>(wave) && wave < G::NYW + G::NXW;
+}
+template <class G>
+FL_HD constexpr bool ays_wave(int wave) {
+    return wave >= G::BL0 / 64 ? wave < G::BL0 / 64 + cdiv(G::BOWN, 64) : wave < cdiv(G::UB - G::BOWN, 64);
+}
+template <class G>
+FL_HD constexpr bool f_wave1(int wave) {   // all waves where a scalar branch there measured slower or F pairs its stores
+    return G::FPAIR || (G::HALO == 4 && G::NADJ == 5) || wave * 64 + NT < G::NIN;
+}
+FL_HD constexpr int cmin(int a, int b) { return a < b ? a : b; }
+template <class G>
+FL_HD constexpr int f_lane(int c) {   // with FPAIR a lane without a second column writes into the padding instead
+    return G::FPAIR ? c : cmin(c, G::NIN - 1);
+}
+template <class G>
+FL_HD constexpr int y_lane(int tid) {
+    return cmin(tid, G::YITEMS - 1);
+}
+template <class G>
+FL_HD constexpr int x_lane(int tid) {
+    return cmin(tid, G::XL0 + G::UX - 1);
+}
+template <class G>
+FL_HD constexpr int ays_lane(int tid) {
+    return tid >= G::BL0 ? cmin(tid, G::BL0 + G::BOWN - 1) : cmin(tid, G::UB - G::BOWN - 1);
+}
+
 // F: input column c (lane + j * NT) of the input region, if c < NIN: its position (ix, iy) and
 // the offset of its z-sum in each of the five Zs planes.
 template <class G>
@@ -227,6 +298,18 @@ FL_HD constexpr int ax_wave(int slot) {
     return G::NADJ > 3 ? G::NYW + slot
                        : G::NYW == 6 ? (slot == 0 ? 6 : slot == 1 ? 7 : slot == 2 ? 10 : 11)
                                      : (slot == 0 ? 5 : slot == 1 ? 6 : slot == 2 ? 7 : 9);
+}
+
+template <class G>
+FL_HD constexpr bool a_wave(int wave) {
+    bool a = false;
+    for (int s = 0; s < G::NAW; ++s) a = a || wave == ax_wave<G>(s);
+    return a;
+}
+template <class G>
+FL_HD constexpr int ax_lane(int tid) {
+    constexpr int LAST_WAVE = ax_wave<G>(G::NAW - 1), LAST = LAST_WAVE * 64 + (G::UA - 1) % 64;
+    return (tid >> 6) == LAST_WAVE ? cmin(tid, LAST) : tid;
 }
 
 // AX unit of lane tid (phase P0): sums of one adjoint field over one segment of position pos

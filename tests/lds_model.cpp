@@ -1,20 +1,25 @@
 // Host-side model of the LDS accesses of the fused LNCC kernel (lncc_fused_kernel.h): for every
 // halo h = 1..4 (tile 32 x 32, and 32 x 24 at h = 4), with three adjoint fields (pred gradient)
 // and with five (both gradients), it enumerates the LDS reads and writes of every lane in every
-// stage from the same lane maps the kernel uses (lncc_geometry.h) and checks
+// stage from the same role waves, repeated lanes and lane maps the kernel uses (lncc_geometry.h) and
+// checks
+//   roles     every lane of a role's waves has a unit, and no wave two kinds of unit in one phase
+//             (with five adjoint fields AYs units may run on Y waves);
 //   bounds    every access lies inside its __shared__ array (spare floats included);
-//   races     within a phase no address is written twice, and no array written in a phase is read
-//             in it (the two phases are separated by the workgroup barriers);
+//   races     within a phase no address is written by two units (lanes past a role's last unit
+//             repeat that unit, the same values to the same addresses), and no array written in a
+//             phase is read in it (the two phases are separated by the workgroup barriers);
 //   coverage  every read that feeds a used output (one inside the adjoint region or the output
 //             tile) reads an address the producing stage writes, and each used output's window is
 //             inside what its lane reads.
 // ROCm has no LDS race checker and GPU address sanitizers do not cover LDS, so this stands in
 // for the compute-sanitizer workloads of the reference (tests/_sanitize*.py).
 //
-// Usage: lds_model [plant]. plant = 0 checks the kernel's maps; 1..4 plant one mistake in the
+// Usage: lds_model [plant]. plant = 0 checks the kernel's maps; 1..7 plant one mistake in the
 // model's view of them (F writes one column too far, Y rows one float short, AYs stores with a
-// row stride one too small, X rows read past their buffer), which must be reported. Prints one
-// line per configuration and exits 0 when every check passes.
+// row stride one too small, X rows read past their buffer, lanes past the last X unit not sent to
+// it, lanes sent to the last Y item but one, an X wave too many), which must be reported. Prints
+// one line per configuration and exits 0 when every check passes.
 #include <cstdio>
 #include <cstdlib>
 #include <set>
@@ -33,7 +38,7 @@ struct Model {
     long failures = 0;
     std::string cfg;
     std::vector<long> size;
-    // per phase: addresses written per array (with multiplicity), arrays read
+    // per phase: the unit that wrote each address of each array (0 = none), arrays read
     std::vector<std::vector<int>> writes[2];
     std::set<int> read_arrays[2];
     std::set<int> written_arrays[2];
@@ -42,12 +47,15 @@ struct Model {
         if (failures < 8) std::printf("  FAIL %s: %s\n", cfg.c_str(), what.c_str());
         ++failures;
     }
-    void write(int phase, int arr, long addr) {
+    void write(int phase, int arr, long addr, int unit) {
         if (addr < 0 || addr >= size[arr]) {
             fail(std::string("write out of ") + kName[arr] + " at " + std::to_string(addr));
             return;
         }
-        writes[phase][arr][addr] += 1;
+        int& by = writes[phase][arr][addr];
+        if (by != 0 && by != unit + 1)
+            fail(std::string("address written twice in one phase: ") + kName[arr] + "[" + std::to_string(addr) + "]");
+        by = unit + 1;
         written_arrays[phase].insert(arr);
     }
     void read(int phase, int arr, long addr, int len) {
@@ -85,70 +93,99 @@ long check(int plant) {
     const int rows_y = fl::row_read(G::SY + 2 * H) - (plant == 2 ? 1 : 0);
     const int rows_b = fl::row_read(G::SB + 2 * H);
 
+    // ---- the roles of a lane, and the lane whose unit it takes
+    struct Lane {
+        bool y, x, b, a, f1;
+        int y_lane, x_lane, b_lane, a_lane;
+    };
+    auto lane_of = [&](int tid) {
+        const int wave = tid >> 6;
+        Lane l;
+        l.y = fl::y_wave<G>(wave);
+        l.x = fl::x_wave<G>(wave) || (plant == 7 && wave == G::NYW + G::NXW);
+        l.b = fl::ays_wave<G>(wave);
+        l.a = fl::a_wave<G>(wave);
+        l.f1 = fl::f_wave1<G>(wave);
+        l.y_lane = plant == 6 ? fl::cmin(tid, G::YITEMS - 2) : fl::y_lane<G>(tid);
+        l.x_lane = plant == 5 ? tid : fl::x_lane<G>(tid);
+        l.b_lane = fl::ays_lane<G>(tid);
+        l.a_lane = fl::ax_lane<G>(tid);
+        return l;
+    };
     // ---- writes of both phases first (each phase's reads use the other phase's writes)
     for (int tid = 0; tid < fl::NT; ++tid) {
+        const Lane l = lane_of(tid);
+        const std::string who = "lane " + std::to_string(tid);
         // P0 / F: the five z-sums of each input column
         for (int j = 0; j < G::J; ++j) {
+            if (j > 0 && !l.f1) {
+                if (tid + j * fl::NT < G::NIN) m.fail(who + " skips an input column");
+                continue;
+            }
+            const int c = fl::f_lane<G>(tid + j * fl::NT);
             int ix, iy, zaddr;
-            if (!fl::f_column<G>(tid + j * fl::NT, ix, iy, zaddr)) {
-                if (!G::FPAIR) continue;
+            if (!fl::f_column<G>(c, ix, iy, zaddr)) {
+                if (!G::FPAIR) {
+                    m.fail(who + " has no input column");
+                    continue;
+                }
                 // paired stores: a lane without this column writes zeros into the plane padding
-                int ix0, iy0;
-                fl::f_column<G>(tid, ix0, iy0, zaddr);
+                fl::f_column<G>(tid, ix, iy, zaddr);
                 zaddr += j * fl::NT;
                 if (zaddr < G::IY * G::ZS) m.fail("F padding write inside the plane");
             }
             if (plant == 1) zaddr += 1;
-            for (int q = 0; q < 5; ++q) m.write(0, ZS, (long)q * G::ZP + zaddr);
+            for (int q = 0; q < 5; ++q) m.write(0, ZS, (long)q * G::ZP + zaddr, c);
         }
         // P1 / Y: the NA adjoint fields of SY outputs of column ax
-        if (tid < G::YITEMS) {
+        if (l.y) {
             int seg, ax, xs, gs;
-            fl::y_item<G>(tid, seg, ax);
-            fl::y_offsets<G>(tid, xs, gs);  // the kernel's per-lane form of the same addresses
+            if (l.y_lane >= G::YITEMS) m.fail(who + " has no Y item");
+            fl::y_item<G>(l.y_lane, seg, ax);
+            fl::y_offsets<G>(l.y_lane, xs, gs);  // the kernel's per-lane form of the same addresses
             for (int c = 0; c < NA; ++c)
                 for (int i = 0; i < G::SY; ++i) {
                     const int a = gs + c * G::GP + i * G::GST;
                     if (a != fl::y_gs<G>(c, ax, seg * G::SY + i)) m.fail("Y offsets disagree with y_gs");
-                    m.write(1, GS, a);
+                    m.write(1, GS, a, l.y_lane);
                 }
         }
-        // P1 / AYs
-        int bsrc, bdst;
-        if (fl::ays_unit<G>(tid, bsrc, bdst))
-            for (int i = 0; i < G::SB; ++i) m.write(1, GY, bdst + (long)i * (G::BW - (plant == 3 ? 1 : 0)));
-        // P1 / X, P0 / AX
         int src, dst;
-        if (fl::x_unit<G>(tid, src, dst))
-            for (int i = 0; i < G::SX; ++i) m.write(1, XS, dst + (long)i * G::XS);
-        if (fl::ax_unit<G>(tid, src, dst))
-            for (int i = 0; i < G::SA; ++i) m.write(0, GXS, dst + (long)i * G::GXS);
-        // lane kinds: a lane has at most one of Y, X, AYs (P1; with five adjoint fields the AYs
-        // units run on Y lanes after Y's arithmetic, which reads no LDS row) and at most one of
-        // Y, AX (P0)
-        int s2, d2;
-        const bool y = tid < G::YITEMS, x = fl::x_unit<G>(tid, s2, d2), b = fl::ays_unit<G>(tid, s2, d2);
-        const bool two_p1 = (x && (y || b)) || (y && b && !G::B_ON_Y);
-        const int p0 = y + fl::ax_unit<G>(tid, s2, d2);
-        if (two_p1 || p0 > 1) m.fail("lane " + std::to_string(tid) + " has two units in one phase");
+        // P1 / AYs
+        if (l.b) {
+            if (fl::ays_unit<G>(l.b_lane, src, dst))
+                for (int i = 0; i < G::SB; ++i) m.write(1, GY, dst + (long)i * (G::BW - (plant == 3 ? 1 : 0)), l.b_lane);
+            else
+                m.fail(who + " has no AYs unit");
+        }
+        // P1 / X, P0 / AX
+        if (l.x) {
+            if (fl::x_unit<G>(l.x_lane, src, dst))
+                for (int i = 0; i < G::SX; ++i) m.write(1, XS, dst + (long)i * G::XS, l.x_lane);
+            else
+                m.fail(who + " has no X unit");
+        }
+        if (l.a) {
+            if (fl::ax_unit<G>(l.a_lane, src, dst))
+                for (int i = 0; i < G::SA; ++i) m.write(0, GXS, dst + (long)i * G::GXS, l.a_lane);
+            else
+                m.fail(who + " has no AX unit");
+        }
+        // kinds: a lane has at most one of Y, X, AYs (P1; with five adjoint fields the AYs units run
+        // on Y lanes after Y's arithmetic, which reads no LDS row) and at most one of Y, AX (P0)
+        if ((l.x && (l.y || l.b)) || (l.y && l.b && !G::B_ON_Y) || (l.y && l.a))
+            m.fail(who + " has two units in one phase");
     }
-    // ---- races: one write per address per phase
-    for (int p = 0; p < 2; ++p)
-        for (int a = 0; a < NARR; ++a)
-            for (long x = 0; x < m.size[a]; ++x)
-                if (m.writes[p][a][x] > 1) {
-                    m.fail(std::string("address written twice in one phase: ") + kName[a] + "[" + std::to_string(x) + "]");
-                    break;
-                }
 
     // ---- reads, and the reads that feed used outputs
     long used_outputs = 0;
     for (int tid = 0; tid < fl::NT; ++tid) {
+        const Lane l = lane_of(tid);
         // P0 / Y reads rows of Xs; outputs ay < AY are used, each reading its 2h+1 window
-        if (tid < G::YITEMS) {
+        if (l.y) {
             int seg, ax, xs, gs;
-            fl::y_item<G>(tid, seg, ax);
-            fl::y_offsets<G>(tid, xs, gs);
+            fl::y_item<G>(l.y_lane, seg, ax);
+            fl::y_offsets<G>(l.y_lane, xs, gs);
             const int y0 = seg * G::SY;
             if (xs != ax * G::XS + y0) m.fail("Y row offset disagrees with the item");
             for (int q = 0; q < 5; ++q) {
@@ -163,17 +200,16 @@ long check(int plant) {
             }
         }
         // P1 / AYs reads rows of GXs; every output oy < TY is used
-        int bsrc, bdst;
-        if (fl::ays_unit<G>(tid, bsrc, bdst)) {
-            m.read(1, GXS, bsrc, rows_b);
+        int src, dst;
+        if (l.b && fl::ays_unit<G>(l.b_lane, src, dst)) {
+            m.read(1, GXS, src, rows_b);
             for (int i = 0; i < G::SB; ++i) {
-                m.used(1, GXS, bsrc + i, 2 * H + 1);
+                m.used(1, GXS, src + i, 2 * H + 1);
                 ++used_outputs;
             }
         }
         // P1 / X reads rows of Zs (outputs ax < AX used), P0 / AX reads rows of Gs (all used)
-        int src, dst;
-        if (fl::x_unit<G>(tid, src, dst)) {
+        if (l.x && fl::x_unit<G>(l.x_lane, src, dst)) {
             const long s = src + (plant == 4 ? 5L * G::ZP : 0);
             m.read(1, ZS, s, rows_x);
             const int start = (dst % G::XP) / G::XS;  // first output position of the segment
@@ -183,7 +219,7 @@ long check(int plant) {
                 ++used_outputs;
             }
         }
-        if (fl::ax_unit<G>(tid, src, dst)) {
+        if (l.a && fl::ax_unit<G>(l.a_lane, src, dst)) {
             m.read(0, GS, src, rows_a);
             for (int i = 0; i < G::SA; ++i) {
                 if (i + 2 * H + 1 > rows_a) m.fail("AX window past the row read");

@@ -44,3 +44,10 @@ def test_kernel_lane_maps_pass(model):
 def test_planted_mistakes_are_reported(model, plant, kind):
     r = subprocess.run([model, str(plant)], capture_output=True, text=True)
     assert r.returncode == 1 and kind in r.stdout, r.stdout
+
+
+@pytest.mark.parametrize("plant,kind", [(5, "has no X unit"), (6, "used read of unwritten Gs"),
+                                        (7, "has two units in one phase")])
+def test_planted_role_mistakes_are_reported(model, plant, kind):
+    r = subprocess.run([model, str(plant)], capture_output=True, text=True)
+    assert r.returncode == 1 and kind in r.stdout, r.stdout
