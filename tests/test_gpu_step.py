@@ -4,6 +4,7 @@ import contextlib
 
 import pytest
 import torch
+import torch.utils.checkpoint
 
 import fused_lncc
 import workloads as wl
@@ -135,6 +136,90 @@ def test_hooks_create_graph_and_streams(monkeypatch):
             side.backward()
         torch.cuda.current_stream().wait_stream(s)
         return (torch.tensor(len(seen)), again.detach(), torch.tensor(again.requires_grad), side.detach(), p.grad)
+    for a, b in zip(*both(monkeypatch, f)):
+        same(a, b)
+
+
+def checkpointed(reentrant):
+    def f():
+        p, t = pair()
+        p.requires_grad_(True)
+        loss = torch.utils.checkpoint.checkpoint(lambda x: fused_lncc_loss(2.0 * x, t, 7), p, use_reentrant=reentrant)
+        loss.backward()
+        return loss.detach(), p.grad
+    return f
+
+
+def checkpointed_retained():
+    """The second backward needs the saved inputs, which the checkpoint forms again."""
+    p, t = pair()
+    p.requires_grad_(True)
+    loss = torch.utils.checkpoint.checkpoint(lambda x: fused_lncc_loss(2.0 * x, t, 7), p, use_reentrant=False)
+    return torch.autograd.grad(loss, p, retain_graph=True) + torch.autograd.grad(loss, p)
+
+
+def anomaly_mode():
+    p, t = pair()
+    with torch.autograd.detect_anomaly(check_nan=True):
+        loss = fused_lncc_loss(p.requires_grad_(True), t, 7)
+        loss.backward()
+        bad = fused_lncc_loss(p, torch.full_like(t, float("nan")), 7)
+        assert torch.isnan(bad).item()
+        with pytest.raises(RuntimeError, match="nan values"):
+            torch.autograd.grad(bad, p)
+    return loss.detach(), p.grad
+
+
+def inference_mode():
+    p, t = pair()
+    with torch.inference_mode():
+        loss = fused_lncc_loss(p.requires_grad_(True), t, 7)
+        assert loss.is_inference() and not loss.requires_grad
+        u = t.clone()   # an inference tensor: no graph can save it
+    with pytest.raises(RuntimeError, match="Inference tensors cannot be saved"):
+        fused_lncc_loss(p, u, 7)
+    return (loss.clone(),)
+
+
+def compiled_autograd():
+    from torch._dynamo import compiled_autograd as ca
+    p, t = pair()
+    loss = fused_lncc_loss(p.requires_grad_(True), t, 7)
+    graphs = []
+    with ca._enable(lambda gm: (graphs.append(gm), torch.compile(gm, backend="eager"))[1]):
+        loss.backward()
+    assert len(graphs) == 1
+    return loss.detach(), p.grad
+
+
+@pytest.mark.filterwarnings("ignore:Anomaly Detection:UserWarning", "ignore:Error detected:UserWarning")
+@pytest.mark.parametrize("f", [checkpointed(False), checkpointed(True), checkpointed_retained, anomaly_mode, inference_mode,
+                               compiled_autograd], ids=lambda f: f.__qualname__.split(".")[0])
+def test_autograd_modes(monkeypatch, f):
+    for a, b in zip(*both(monkeypatch, f)):
+        same(a, b)
+
+
+def test_threads(monkeypatch):
+    """Forward and backward from several threads at once, each with its own inputs."""
+    import threading
+
+    def f():
+        out = [None] * 4
+
+        def work(i):
+            p, t = pair(seed=i)
+            p.requires_grad_(True)
+            for _ in range(10):
+                p.grad = None
+                fused_lncc_loss(p, t, 7).backward()
+            out[i] = p.grad
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+        for th in threads:
+            th.start()
+        for th in threads:
+            th.join()
+        return out
     for a, b in zip(*both(monkeypatch, f)):
         same(a, b)
 
