@@ -130,18 +130,25 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
         }
     }
     if constexpr (G::FPAIR) zaddr[1] = zaddr[0] + NT;
-    const bool f_col1 = f_wave1<G>(wave_id);   // this wave has second columns
+    const bool f_col1 = G::F_ALL || wave_id * 64 + NT < G::NIN;   // this wave has second columns
     // Y items on lanes [0, YITEMS) (y-sums in P0, ncc arithmetic in P1), X and AYs units in P1,
     // AX units in P0 (lncc_geometry.h); offsets into the source and destination buffers
     // (a lane has at most one unit of X and AYs, so the two share one pair of offsets; with five
     // adjoint fields the AYs units sit on Y lanes)
-    // The roles are whole waves, so that a stage is entered through one scalar compare and branch.
-    const bool wave_y = y_wave<G>(wave_id), wave_x = x_wave<G>(wave_id), wave_b = ays_wave<G>(wave_id),
-               wave_a = a_wave<G>(wave_id);
+    // The roles are whole waves, a lane past a role's last unit repeats it (lncc_geometry.h).
+    const bool wave_y = wave_id < G::NYW;
+    const bool wave_x = !wave_y && wave_id < G::NYW + G::NXW;
+    const bool wave_b = wave_id >= G::BL0 / 64 ? wave_id < G::BL0 / 64 + G::NBW : wave_id < G::NBYW;
+    bool wave_a = false;
+#pragma unroll
+    for (int sl = 0; sl < G::NAW; ++sl) wave_a = wave_a || wave_id == ax_wave<G>(sl);
     int u_src = 0, u_dst = 0, a_src, a_dst;
-    x_unit<G>(x_lane<G>(tid), u_src, u_dst);
-    ax_unit<G>(ax_lane<G>(tid), a_src, a_dst);
-    if (wave_b) ays_unit<G>(ays_lane<G>(tid), u_src, u_dst);
+    x_unit<G>(min(tid, G::X_LAST), u_src, u_dst);
+    {
+        constexpr int LAST = ax_last<G>();
+        ax_unit<G>((tid >> 6) == ax_wave<G>(G::NAW - 1) ? min(tid, LAST) : tid, a_src, a_dst);
+    }
+    if (wave_b) ays_unit<G>(tid >= G::BL0 ? min(tid, G::B_LAST) : min(tid, G::BY_LAST), u_src, u_dst);
     int y_seg = 0, y_ax = 0;  // rows seg of AX positions
     // the Y item's offsets into Xs and Gs. At k = 7 they take the registers of the X / AYs unit
     // offsets (a Y lane has no such unit), which with three of Y's rows in flight across F is
@@ -150,7 +157,7 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
     constexpr bool Y_SHARE = HH == 3 && !DUAL;
     int y_xs = 0, y_gs0 = 0;
     if (wave_y) {
-        const int item = y_lane<G>(tid);
+        const int item = min(tid, G::Y_LAST);
         y_item<G>(item, y_seg, y_ax);
         if constexpr (Y_SHARE)
             y_offsets<G>(item, u_src, u_dst);
@@ -371,11 +378,11 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
     //  * Both gradients (five adjoint fields, fourteen more ring registers per lane at k = 7):
     //    fewer early rows, all five at k = 3, two (bf16) or none (fp32) at k = 5, none above, and no
     //    AX row before F. At k = 9 the two 9-plane rings and the five adjoint rings exceed the 128
-    //    registers even so: 36-54 spill to scratch, and the launch still runs a quarter faster than
-    //    two pred-gradient passes.
-    // What a step costs: 16 waves, 4 per SIMD, none of VALU issue (~55% of the step), LDS (58% active)
+    //    registers even so: 36 (fp32) or 50 (bf16) spill to scratch, and the launch still runs a quarter
+    //    faster than two pred-gradient passes. At k = 7 two or four do.
+    // What a step costs: 16 waves, 4 per SIMD, none of VALU issue (~55% of the step), LDS (61% active)
     // or HBM (25%) saturated. A scalar instruction takes an issue cycle of its wave like a vector one,
-    // and a step had 92 of them for 149 vector ones: lane masks for roles that are whole waves, and
+    // and a step had 77 of them for 149 vector ones: lane masks for roles that are whole waves, and
     // five buffer resources rebuilt from 64-bit addresses. Roles as scalar branches and addresses
     // advanced in place leave about 55; with the row waits moved behind F, (2,16,128^3) went from
     // 0.344 / 0.369 / 0.401 / 0.584 to 0.331 / 0.359 / 0.391 / 0.564 ms at k = 3 / 5 / 7 / 9.
@@ -383,7 +390,10 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
                                  : HH <= 1 ? 5 : HH == 2 ? 3 : HH == 3 ? 2 : 0;   // Y rows read before F
     constexpr bool F_STORE_AT_ONCE = Y_EARLY < 5;
     // no z-sums for the drain steps, which X does not read (2-5% at k >= 5; at k = 3 1% slower, and both
-    // gradients at k = 9, which spill, 8%)
+    // gradients at k = 9, which spill, 8%). What it costs: with the branch around F in the march, taken or
+    // not, float32 planes of 256 x 256 at k = 7 are read from HBM 1.6 times instead of 1.05 (AZ's re-read
+    // misses the L2): (2,16,256^3) 3.00 -> 3.09 ms, both gradients 3.71 -> 3.79; (1,1,160,192,224) 55.2
+    // -> 54.2 us, 96^3 21.4 -> 20.8, bfloat16 faster at every size.
     constexpr bool F_STOP = HH >= 2 && !(DUAL && HH == 4);
     constexpr bool AX_EARLY = HH <= 2 && !DUAL;               // the AX row read before F
     constexpr int NY = G::SY + 2 * HH, NA = G::SA + 2 * HH, NX = G::SX + 2 * HH, NB = G::SB + 2 * HH;
@@ -468,10 +478,10 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void lncc_fused_kernel(FusedArgs a) 
                 // last use of those lines. With the default policy both would be promoted in the
                 // L2 and push out the planes that F loaded and this stage re-reads 2h+3 steps
                 // later, so that every input byte would be fetched about twice; marked
-                // evict-first, every input byte is fetched from HBM once. bf16 gradient rows of a
-                // tile are half a 128-byte line (the x-neighbour tile writes the other half):
-                // those stores keep the default policy, so that the L2 merges the two halves into
-                // one write.
+                // evict-first, every input byte is fetched from HBM once at (2,16,128^3) (float32
+                // planes of 256 x 256: F_STOP above). bf16 gradient rows of a tile are half a
+                // 128-byte line (the x-neighbour tile writes the other half): those stores keep the
+                // default policy, so that the L2 merges the two halves into one write.
                 const uint32_t gb = zo >= z0 ? plane_bytes : 0u;   // zo < z1 up to the march's last step
                 store_elem_buf<BF16, BF16 ? 0 : kNT>(words_at(oga, gb), z_voff, g);
                 oga += PB;

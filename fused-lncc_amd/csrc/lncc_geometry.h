@@ -1,7 +1,7 @@
 // Tile geometry and per-lane work maps of the LNCC kernels. Plain C++ (no HIP builtins): the kernels
-// take their roles and every LDS offset they use from these functions, and the host-side models of
+// take the bounds of their roles and every LDS offset they use from here, and the host-side models of
 // their LDS accesses (tests/lds_model.cpp, forward_lds_model.cpp, small_lds_model.cpp) enumerate the
-// same functions for every lane.
+// same for every lane.
 #pragma once
 
 #if defined(__HIPCC__)
@@ -97,6 +97,13 @@ struct Geo {
     static constexpr int NYW = cdiv(YITEMS, 64), XL0 = 64 * NYW, NXW = cdiv(UX, 64), BL0 = rup64(XL0 + UX), NAW = cdiv(UA, 64);
     static constexpr int BOWN = UB < NT - BL0 ? UB : NT - BL0;
     static constexpr bool B_ON_Y = UB > BOWN;
+    // The roles are whole waves, so that a stage is entered through one scalar branch: Y on waves [0, NYW),
+    // X on the next NXW, AYs on NBW from lane BL0 on and NBYW from lane 0 on, AX on ax_wave(0..NAW-1), F's
+    // second columns on waves that reach below NIN (or on all: where F pairs its stores, and where a scalar
+    // branch measured slower). A lane past the last unit of a role's last wave repeats that unit, the same
+    // values to the same addresses, so that no stage needs a lane mask: the lanes of those units.
+    static constexpr int NBW = cdiv(BOWN, 64), NBYW = cdiv(UB - BOWN, 64);
+    static constexpr int Y_LAST = YITEMS - 1, X_LAST = XL0 + UX - 1, B_LAST = BL0 + BOWN - 1, BY_LAST = UB - BOWN - 1;
     // Y items and X units on disjoint lanes, AYs units on lanes of their own or on Y lanes (the
     // kernel keeps a Y item's offsets in the registers of the X / AYs unit offsets at k = 7 with
     // three adjoint fields)
@@ -122,6 +129,7 @@ struct Geo {
     // 2 NT floats: a lane without a second column writes its (zero) z-sums into the padding, so
     // that every lane's ten z-sum stores pair into five write2st64
     static constexpr bool FPAIR = (H == 3 && ZS == IX && J == 2);
+    static constexpr bool F_ALL = FPAIR || (H == 4 && NA == 5);   // second F columns on all waves
     static constexpr int ZP = FPAIR ? 2 * NT : H >= 2 ? rup64(IY * ZS) : IY * ZS, XP = XR * XS, GP = (ASWAP ? AX : YR) * GS, GXP = (ASWAP ? TY : TX) * GXS,
                          GYP = H >= 2 ? rup64(TY * GYS) : TY * GYS;
     // A segment reads row_read(S + 2H) floats from its start; reads past a row's end stay inside
@@ -225,43 +233,11 @@ FL_HD inline void split32(int idx, int n_rows, int& row, int& pos) {
     }
 }
 
-// The plane-marching kernel's roles are whole waves: which waves take Y items (y-sums in P0, ncc
-// arithmetic in P1), X units, AYs units (P1; with five adjoint fields some of them on Y waves) and AX
-// units (P0), and which have second F columns. A lane past the last unit of a role's last wave repeats
-// that unit, the same values to the same addresses, so that no stage needs a lane mask: *_lane gives the
-// lane whose unit a lane of the role takes (f_lane the input column).
+// The input column that a lane's column slot c (lane + j * NT) takes: a slot past the last column
+// repeats it; with FPAIR such a lane writes into the padding of the Zs planes instead.
 template <class G>
-FL_HD constexpr bool y_wave(int wave) {
-    return wave < G::NYW;
-}
-template <class G>
-FL_HD constexpr bool x_wave(int wave) {
-    return !y_wave<G>(wave) && wave < G::NYW + G::NXW;
-}
-template <class G>
-FL_HD constexpr bool ays_wave(int wave) {
-    return wave >= G::BL0 / 64 ? wave < G::BL0 / 64 + cdiv(G::BOWN, 64) : wave < cdiv(G::UB - G::BOWN, 64);
-}
-template <class G>
-FL_HD constexpr bool f_wave1(int wave) {   // all waves where a scalar branch there measured slower or F pairs its stores
-    return G::FPAIR || (G::HALO == 4 && G::NADJ == 5) || wave * 64 + NT < G::NIN;
-}
-FL_HD constexpr int cmin(int a, int b) { return a < b ? a : b; }
-template <class G>
-FL_HD constexpr int f_lane(int c) {   // with FPAIR a lane without a second column writes into the padding instead
-    return G::FPAIR ? c : cmin(c, G::NIN - 1);
-}
-template <class G>
-FL_HD constexpr int y_lane(int tid) {
-    return cmin(tid, G::YITEMS - 1);
-}
-template <class G>
-FL_HD constexpr int x_lane(int tid) {
-    return cmin(tid, G::XL0 + G::UX - 1);
-}
-template <class G>
-FL_HD constexpr int ays_lane(int tid) {
-    return tid >= G::BL0 ? cmin(tid, G::BL0 + G::BOWN - 1) : cmin(tid, G::UB - G::BOWN - 1);
+FL_HD constexpr int f_lane(int c) {
+    return G::FPAIR || c < G::NIN ? c : G::NIN - 1;
 }
 
 // F: input column c (lane + j * NT) of the input region, if c < NIN: its position (ix, iy) and
@@ -300,16 +276,10 @@ FL_HD constexpr int ax_wave(int slot) {
                                      : (slot == 0 ? 5 : slot == 1 ? 6 : slot == 2 ? 7 : 9);
 }
 
+// The last lane with an AX unit, on the last of those waves.
 template <class G>
-FL_HD constexpr bool a_wave(int wave) {
-    bool a = false;
-    for (int s = 0; s < G::NAW; ++s) a = a || wave == ax_wave<G>(s);
-    return a;
-}
-template <class G>
-FL_HD constexpr int ax_lane(int tid) {
-    constexpr int LAST_WAVE = ax_wave<G>(G::NAW - 1), LAST = LAST_WAVE * 64 + (G::UA - 1) % 64;
-    return (tid >> 6) == LAST_WAVE ? cmin(tid, LAST) : tid;
+FL_HD constexpr int ax_last() {
+    return ax_wave<G>(G::NAW - 1) * 64 + (G::UA - 1) % 64;
 }
 
 // AX unit of lane tid (phase P0): sums of one adjoint field over one segment of position pos

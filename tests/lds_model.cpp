@@ -20,6 +20,7 @@
 // row stride one too small, X rows read past their buffer, lanes past the last X unit not sent to
 // it, lanes sent to the last Y item but one, an X wave too many), which must be reported. Prints
 // one line per configuration and exits 0 when every check passes.
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <set>
@@ -101,15 +102,16 @@ long check(int plant) {
     auto lane_of = [&](int tid) {
         const int wave = tid >> 6;
         Lane l;
-        l.y = fl::y_wave<G>(wave);
-        l.x = fl::x_wave<G>(wave) || (plant == 7 && wave == G::NYW + G::NXW);
-        l.b = fl::ays_wave<G>(wave);
-        l.a = fl::a_wave<G>(wave);
-        l.f1 = fl::f_wave1<G>(wave);
-        l.y_lane = plant == 6 ? fl::cmin(tid, G::YITEMS - 2) : fl::y_lane<G>(tid);
-        l.x_lane = plant == 5 ? tid : fl::x_lane<G>(tid);
-        l.b_lane = fl::ays_lane<G>(tid);
-        l.a_lane = fl::ax_lane<G>(tid);
+        l.y = wave < G::NYW;
+        l.x = !l.y && wave < G::NYW + G::NXW + (plant == 7 ? 1 : 0);
+        l.b = wave >= G::BL0 / 64 ? wave < G::BL0 / 64 + G::NBW : wave < G::NBYW;
+        l.a = false;
+        for (int s = 0; s < G::NAW; ++s) l.a = l.a || wave == fl::ax_wave<G>(s);
+        l.f1 = G::F_ALL || wave * 64 + fl::NT < G::NIN;
+        l.y_lane = std::min(tid, G::Y_LAST - (plant == 6 ? 1 : 0));
+        l.x_lane = plant == 5 ? tid : std::min(tid, G::X_LAST);
+        l.b_lane = tid >= G::BL0 ? std::min(tid, G::B_LAST) : std::min(tid, G::BY_LAST);
+        l.a_lane = wave == fl::ax_wave<G>(G::NAW - 1) ? std::min(tid, fl::ax_last<G>()) : tid;
         return l;
     };
     // ---- writes of both phases first (each phase's reads use the other phase's writes)
