@@ -162,7 +162,7 @@ def main():
     stream = torch.cuda.current_stream(dev)
 
     def kernel():
-        if a.target_grad:   # both gradients: the one fused launch (k <= 7) and the loss finalize
+        if a.target_grad:   # both gradients: the one fused launch and the loss finalize
             _lib.check(lib.fl_lncc_loss_grad_pt(p.data_ptr(), t.data_ptr(), code, B, D, H, W, k, 1e-5,
                                                 loss_buf.data_ptr(), grad.data_ptr(), grad_t.data_ptr(),
                                                 ws.data_ptr(), nbytes, stream.cuda_stream))

@@ -49,9 +49,10 @@ int device_cus() {
     return n;
 }
 
-// Workgroups: B volumes x (W/TX) x (H/TY) tiles x D-chunks. A chunk of d output planes costs
-// d + 2h + 4 pipeline steps (it recomputes the halo planes of its neighbours), so D is split only
-// where that shortens the launch: small volumes, whose tiles alone leave CUs idle, get short chunks.
+// Workgroups: B volumes x (W/TX) x (H/TY) tiles x D-chunks. A chunk of d output planes takes
+// d + 2h + 3 pipeline steps (it recomputes the halo planes of its neighbours; h fewer at a volume's
+// first planes) after the loads of its first window, counted as one more, so D is split only where
+// that shortens the launch: small volumes, whose tiles alone leave CUs idle, get short chunks.
 // fl_test_set_dchunk fixes the chunk length for the calling thread (tests of chunk seams and of
 // long unsplit marches).
 Plan plan_fused(int64_t B, int64_t D, int64_t H, int64_t W, int halo) {
@@ -71,8 +72,8 @@ Plan plan_fused(int64_t B, int64_t D, int64_t H, int64_t W, int halo) {
     // callers pass shapes that passed check_grid, so base < 2^32 / NT; a forced chunk length can
     // multiply it by up to D <= 2^30, which still fits int64
     const int64_t base = B * p.ntx * p.nty;
-    // Split D into nzc chunks. A chunk of d planes costs d + 2h + 4 pipeline steps, and the
-    // workgroups run in rounds of one per CU: pick the split with the fewest rounds x steps (ties:
+    // Split D into nzc chunks. A chunk of d planes costs d + 2h + 4 steps (above), and the workgroups
+    // run in rounds of one per CU: pick the split with the fewest rounds x steps (ties:
     // fewer workgroups).
     const int64_t kCUs = device_cus();
     int64_t best_cost = -1, dchunk = D;

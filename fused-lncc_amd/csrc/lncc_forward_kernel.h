@@ -19,10 +19,11 @@
 // Window sums, formula, clamp, NaN policy and range scale are those of lncc_fused_kernel.h: every
 // sum is one of its window's own values.
 //
-// Bound: VALU issue. At k = 7 a plane of a 48 x 32 tile takes ~2150 cycles of a CU, of which its vector
-// instructions fill ~1550 per SIMD (additions and products issue in 2.3 cycles, DPP additions, max,
-// compares and selects in 4.2, the reciprocal in 8); the LDS is busy for ~800, HBM fetches each input
-// byte 1.005 times. At (2,16,128^3) fp32: 0.219 / 0.242 / 0.281 / 0.452 ms -> 0.150 / 0.164 / 0.179 /
+// Bound: VALU issue. At k = 7 a plane of a 48 x 32 tile takes 2045 cycles of a CU (counters at
+// (2,16,128^3)); its 115 vector instructions a wave fill ~1550 of them per SIMD at their measured issue
+// rates (additions and products 2.3 cycles, DPP additions, max, compares and selects 4.2, the reciprocal
+// 8), 91% as SQ_ACTIVE_INST_VALU counts them (four cycles each); the LDS is active for 862; HBM fetches
+// 1.036 / 1.056 / 1.076 / 1.100 times the input bytes at k = 3 / 5 / 7 / 9. At (2,16,128^3) fp32: 0.219 / 0.242 / 0.281 / 0.452 ms -> 0.150 / 0.164 / 0.179 /
 // 0.216 ms at k = 3 / 5 / 7 / 9 against the gradient kernel run without its adjoint, whose x pass
 // goes through LDS and whose tile carries the adjoint's halo (3.0 TB/s of 8 B per voxel at k = 7);
 // the map of 160x192x224 at k = 9 0.0556 -> 0.0356 ms. F is the longer role and has the lower wave
@@ -98,7 +99,7 @@ __device__ __forceinline__ float field_add(float s, float p, float t) {
 // i + grid, ... in turn. The pieces of one chunk index lie side by side, so that the workgroups
 // running at one time march through neighbouring tiles at the same plane and share their halo
 // columns in the L2 (an even split of the planes over the grid, whose shares start at different
-// planes, fetched 1.48x the input bytes at (2,16,128^3) and gained nothing by its even load).
+// planes, gained nothing by its even load: it fetches the halos again).
 struct Pieces {
     uint32_t i, n, tiles, chunks;
     int D, most;

@@ -48,7 +48,7 @@ hipError_t launch_fused_h3(int mode, bool bf16, const FusedArgs& a, uint32_t nbl
 hipError_t launch_fused_h4(int mode, bool bf16, const FusedArgs& a, uint32_t nblocks, hipStream_t st);
 
 // The forward-only kernel (lncc_forward.hip), MODE_LOSS and MODE_MAPS: `cols` input columns per F lane
-// (forward_width lists the widths of a halo).
+// (3 at every halo, 4 too at halos 1 to 3).
 hipError_t launch_forward(int halo, int cols, int mode, bool bf16, const FusedArgs& a, uint32_t nblocks, hipStream_t st);
 
 // The small-volume kernel (lncc_small.hip): volumes whose D, H and W are all at most kSmallEdge

@@ -1,8 +1,8 @@
 // The fused LNCC kernel for small volumes (each of D, H, W at most 16), gfx950.
 //
-// The plane-marching kernel (lncc_fused_kernel.h) works on 32 x 32 tiles and a D-pipeline of
-// 2h+4 steps: on many small volumes, as in a network's feature maps (the reference benchmarks
-// (1,256,16^3)), three quarters of its lanes idle and the pipeline steps outnumber the planes.
+// The plane-marching kernel (lncc_fused_kernel.h) works on 32 x 32 tiles and takes 2h + 3 pipeline
+// steps beyond the planes of a chunk: on many small volumes, as in a network's feature maps (the
+// reference benchmarks (1,256,16^3)), three quarters of its lanes idle and those steps rival the planes.
 // Here one 1024-lane workgroup holds one whole volume, zero-padded to 16^3, in LDS, and forms the
 // same sums and the same per-voxel arithmetic in four phases separated by workgroup barriers:
 //
